@@ -56,6 +56,14 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 __device__ __forceinline__ bf16x8 ld8(const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 __device__ __forceinline__ float sig(float z) { return 1.f / (1.f + expf(-z)); }
+/* Inference: the hardware's exponential and reciprocal (about 1 ulp each, the
+ * product's rounding adds |z| 2^-24), 4 instructions where the one above is
+ * about 30.  k_infer evaluates 128 of them per sample between BF16 products
+ * of 2^-9 and was bound by them; training keeps the correctly rounded
+ * quotient, whose bits its losses repeat. */
+__device__ __forceinline__ float sig_fast(float z) {
+    return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * z));
+}
 __device__ __forceinline__ f32x4 splat(float v) { return f32x4{v, v, v, v}; }
 
 /* Weights staged per workgroup: BF16 copies for the MFMA operands, FP32 for
@@ -128,7 +136,7 @@ __device__ __forceinline__ void forward(const W& w, L& l, const bf16x8 xa[2], in
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float z = z1[m][t][r];
-                const __bf16 a = (__bf16)(z * sig(z));
+                const __bf16 a = (__bf16)(z * (TRAIN ? sig(z) : sig_fast(z)));
                 const int s = m * 16 + g * 4 + r, k = t * 16 + c;
                 l.a1[s * P64 + k] = a;
                 if constexpr (TRAIN) l.a1t[k * P32 + s] = a;
@@ -152,7 +160,7 @@ __device__ __forceinline__ void forward(const W& w, L& l, const bf16x8 xa[2], in
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float z = acc[r];
-                part[r] += (z * sig(z)) * w3;
+                part[r] += (z * (TRAIN ? sig(z) : sig_fast(z))) * w3;
             }
         }
 #pragma unroll
