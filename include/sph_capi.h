@@ -111,7 +111,10 @@ typedef struct sph_params {
     int32_t precision;
     /* Lanes per particle in the density pass: 0 = one thread per particle
      * (the reference's summation order), 2/4/8/16/32/64 = the particle's cell
-     * box split over that many lanes (same terms, tree-ordered sums). */
+     * box split over that many lanes (same terms, tree-ordered sums).  At 8
+     * (the default), and below small_n_lanes, the pass takes neighbour lists
+     * that a wave builds in place of walking the cells scan by scan: the same
+     * terms, with density_stop 1 the same bits. */
     int32_t density_lanes;
     /* The same for the acceleration pass (0 = one thread per particle). */
     int32_t accel_lanes;
@@ -175,7 +178,8 @@ typedef struct sph_params {
      * lane sums which changes. */
     int32_t near_list_cap;
     /* Every particle active (no slot list) and fewer than this many
-     * particles (0 = off): the density pass takes 32 lanes per particle and
+     * particles (0 = off): the density pass takes 32 lanes per particle (from
+     * its lists, their order of the sums with density_stop 1) and
      * the acceleration pass 16 below 65,536 particles, else 8, in place of
      * density_lanes and accel_lanes.  With one thread (or 8 lanes) per
      * particle such a pass leaves most of the GPU's wave slots empty and

@@ -108,6 +108,8 @@ void destroy_ctx(sph_ctx* ctx) {
     dfree(ctx->pairs_a);
     dfree(ctx->pairs_b);
     dfree(ctx->cell_se);
+    dfree(ctx->block_se[0]);
+    dfree(ctx->block_se[1]);
     dfree(ctx->cell_mark);
     dfree(ctx->tile_hist);
     dfree(ctx->grav_flags);
@@ -116,6 +118,8 @@ void destroy_ctx(sph_ctx* ctx) {
     dfree(ctx->guess);
     dfree(ctx->slot_list);
     dfree(ctx->slot_count);
+    dfree(ctx->redo);
+    dfree(ctx->redo_count);
     dfree(ctx->eos[0]);
     dfree(ctx->eos[1]);
     free_tree(ctx->tree);
@@ -328,6 +332,9 @@ int sph_create(const sph_params* params, const sph_ic_view* ic, const sph_eos_ta
     TRY(dalloc(&ctx->next_active, n));
     TRY(dalloc(&ctx->nr_iters, n));
     TRY(dalloc(&ctx->nr_order, n));
+    TRY(dalloc(&ctx->redo, 2 * n));
+    TRY(dalloc(&ctx->redo_count, 4));
+    TRY(hipMemset(ctx->redo_count, 0, 16));
     TRY(dalloc(&ctx->active, n));
     TRY(dalloc(&ctx->density_work, n));
     TRY(hipMemset(ctx->density_work, 0, 16 * n));
@@ -335,6 +342,8 @@ int sph_create(const sph_params* params, const sph_ic_view* ic, const sph_eos_ta
     TRY(dalloc(&ctx->pairs_a, n));
     TRY(dalloc(&ctx->pairs_b, n));
     TRY(dalloc(&ctx->cell_se, (size_t)ctx->ncells));
+    for (int k = 0; k < 2; ++k)
+        if (params->cell_power >= k + 2) TRY(dalloc(&ctx->block_se[k], (size_t)ctx->ncells >> (3 * (k + 1))));
     TRY(dalloc(&ctx->cell_mark, (size_t)ctx->ncells));
     TRY(hipMemset(ctx->cell_mark, 0, (size_t)ctx->ncells));
     ctx->ntiles = (int)((n + 2047) / 2048);
@@ -594,7 +603,7 @@ int sph_sort(sph_ctx* ctx) {
     ctx->slot_list_valid = false;
     int rc = ctx_begin_pass(ctx, SPH_PASS_SORT);
     if (rc == SPH_OK) rc = launch_sort(ctx);
-    if (rc == SPH_OK) ctx->morton_fresh = true;
+    if (rc == SPH_OK) ctx->morton_fresh = ctx->cells_fresh = true;
     if (rc == SPH_OK) rc = ctx_end_pass(ctx, SPH_PASS_SORT);
     return rc;
 }
@@ -798,6 +807,7 @@ int sph_upload(sph_ctx* ctx, int field, const void* src) {
      * activity replaced: fold with the flags the pass ran under first */
     if (field == SPH_F_ACC) ctx->dv_pending = false;
     if (field == SPH_F_POS || field == SPH_F_VEL || field == SPH_F_MASS) ctx->morton_fresh = false;
+    if (field == SPH_F_POS) ctx->cells_fresh = false;
     if (field == SPH_F_ACTIVE) SPH_TRY_RC(fold_dv(ctx));
     ctx->slot_list_valid = false;
     SPH_HIP_TRY(hipStreamSynchronize(ctx->stream));

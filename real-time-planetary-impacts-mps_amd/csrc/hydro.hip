@@ -23,17 +23,12 @@
  * that membership test and the cache's own range test (r > 2h), which yields
  * the same terms in the same order.
  */
+#include "near_lists.h"
 #include "sph_internal.h"
 
 namespace {
 
 constexpr float kPi1 = 1.f / 3.14159265358979323846f;
-
-struct Cells {
-    const uint2* cell_se;
-    float cell_size;
-    int mask;
-};
 
 /* cellsToScan.h:33-59.  Guard: a non-finite bound gives an empty box and an
  * extent is capped at 2^cell_power cells per axis (the periodic grid), so a
@@ -176,6 +171,11 @@ struct DensityArgs {
     /* every slot: the order in which the groups take them (k_nr_order), or
      * null for slot order */
     const int32_t* order;
+    /* k_density_lists: the slots it leaves to a grouped launch over `redo`
+     * and their count; that launch clears the count the next pass uses */
+    int32_t* redo;
+    int32_t* redo_count;
+    int32_t* clear;
 };
 
 /* Whether the Newton-Raphson iteration goes on after a scan whose relative
@@ -756,6 +756,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LIST ? 7 : 
         if (k < a.n) density_group_particle<G, SPLIT, FLAT, COUNT>(a, a.order ? a.order[k] : k, lane);
         return;
     }
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     const int total = *a.nslots;
     const int nlog = (total + PPB - 1) / PPB;
     const int per = (nlog + kXcds - 1) / kXcds;
@@ -765,6 +766,432 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LIST ? 7 : 
         if (lb >= nlog) break;
         const int e = lb * PPB + g;
         if (e < total) density_group_particle<G, SPLIT, FLAT, COUNT>(a, a.slots[e], lane);
+    }
+}
+
+
+/* The list's radius over the current 2h: how far h may grow before the
+ * lists are built again.  A wider one makes longer lists, and from 1.15 on
+ * many overflow (density pass at 1e6, ms: 1.34 / 1.33 / 1.39 at 1.07 / 1.10 /
+ * 1.13 with the default rule, 2.08 / 2.10 / 2.21 near the fixed point). */
+constexpr float kReachGrow = 1.10f;
+
+__device__ __forceinline__ float clamp01(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, 1.f); }
+/* The spline sum's term w(r / h) m added to `part`, as kW_tp's without its
+ * normalisation: with a = (1 - q/2)+, half of kW_tp's, w = 2 a^3 - b^3; both
+ * truncations are the multiply-add's clamp to [0, 1].  Bit for bit the
+ * grouped pass's (its a is scaled by a power of two). */
+__device__ __forceinline__ float add_w(float part, float r, float m, float k1, float k2) {
+    const float ta = clamp01(fmaf(k2, r, 1.f)), tb = clamp01(fmaf(k1, r, 1.f));
+    const float ta2 = ta * ta, tb2 = tb * tb;
+    return fmaf(fmaf(ta2 + ta2, ta, -(tb2 * tb)), m, part);
+}
+__device__ __forceinline__ float pair_r2(float dx, float dy, float dz) { return fmaf(dz, dz, fmaf(dx, dx, dy * dy)); }
+
+/* The second pass's sums over one lane's entries: kdWdh_tp and
+ * kGradWFactor_tp on shared a and b, with the grouped pass's roundings (q and
+ * a - q are rounded apart there). */
+struct FinalSums {
+    float density_h = 0.f, velDiv = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
+    __device__ __forceinline__ void add(float r, float mass, float dx, float dy, float dz, float4 vj, float4 vi4, float h1) {
+        const float fac = kPi1 * h1 * h1 * h1 * h1, fac_h = -3.f * kPi1 * h1 * h1 * h1 * h1;
+        const float a = fmaxf(fmaf(-h1, r, 2.f), 0.f), b = fmaxf(fmaf(-h1, r, 1.f), 0.f);
+        float aq, bq;
+        {
+#pragma clang fp contract(off)
+            const float q = r * h1;
+            aq = a - q;
+            bq = b - q;
+        }
+        density_h = fmaf(mass, fac_h * fmaf(0.25f * a * a, aq, -(b * b * bq)), density_h);
+        if (r > 1e-12f) {
+            const float r1 = __builtin_amdgcn_rcpf(r);
+            const float vx = vj.x - vi4.x, vy = vj.y - vi4.y, vz = vj.z - vi4.z;
+            const float g = fac * fmaf(3.f * b, b, -0.75f * a * a);
+            const float gx = g * (dx * r1), gy = g * (dy * r1), gz = g * (dz * r1);
+            velDiv = fmaf(mass, fmaf(vz, gz, fmaf(vx, gx, vy * gy)), velDiv);
+            cx = fmaf(mass, fmaf(vy, gz, -(vz * gy)), cx);
+            cy = fmaf(mass, fmaf(vz, gx, -(vx * gz)), cy);
+            cz = fmaf(mass, fmaf(vx, gy, -(vy * gx)), cz);
+        }
+    }
+};
+
+/* density.metal:12-239 for the wave's 64 / GL particles (lane / GL), from
+ * neighbour lists: the candidates within 2h (and a margin) are found once,
+ * each lane keeps its share's distances and masses in registers, and every
+ * Newton-Raphson scan is a sum over them.  The lists are built again when
+ * some h outgrows its margin.  The terms, the stopping rules, the guess's
+ * restart and the neighbour-cache rules are density_group_particle's.
+ *
+ * S = 0: the entries are dealt evenly to the lanes.  S > 0: they are dealt as
+ * density_group_particle<GL S> deals its cells, and every sum has its bits.
+ *
+ * The cell walk (density_group_particle) is bound by VALU issue and by the
+ * latency of its dependent loads: every scan reads the cell table and the
+ * records again, and two candidates in three are beyond 2h or on idle lanes.
+ * From the lists a scan is 6 instructions per entry on registers, bound by
+ * VALU issue alone: of the 24k instructions of a wave of 8 particles at 1e6
+ * near the fixed point (29 scans) about 4k are the entries', 7k the scans'
+ * roots, divisions and control, the rest the lists, deals and second pass.
+ * The pass, walk -> lists, ms: with the default rule 0.72 -> 0.06 at 2e4,
+ * 3.4 -> 1.36 at 1e6, 17 -> 6.1 at 4e6; near the fixed point 2.65 -> 0.41 at
+ * 2e4, 3.39 -> 0.86 at 1e5, 4.94 -> 1.87 at 3e5, 11.4 -> 6.1 at 1e6.
+ *
+ * Particles with more entries than a list (or a bin) holds, or with a
+ * position or an h that is not finite, are left to `redo`. */
+template <int GL, int S, int P>
+__device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, NearLds<GL, S, P>& l) {
+    constexpr int kCap = NearLds<GL, S, P>::kCap;
+    constexpr int NS = S ? S : 1, R = NearLds<GL, S, P>::kRows; /* bins per lane, and their rows in registers */
+    const int lane = (int)(threadIdx.x & 63), gl = lane % GL, g = P == 1 ? 0 : lane / GL;
+    const bool on = index >= 0;
+    if (index == 0 && gl == 0) a.time[1] = a.dt_reset;
+    const uint32_t ind = on ? a.sorted[index].y : 0u;
+    const bool act = on && a.active[ind];
+    const float2* table = on && a.mat[ind] == 400 ? a.eos0 : a.eos1;
+    if (on && !act && !a.skip_inactive && gl == 0) {
+        const float2 pc = eos_sample(table, a.eos_res, a.u[ind], a.rho[ind], a.min_u, a.max_u, a.min_rho, a.max_rho);
+        a.P[ind] = pc.x;
+        a.c[ind] = pc.y;
+        a.nr_iters[ind] = 0;
+    }
+    const float4* __restrict__ spm = a.s_posm;
+    const float4 pm = act ? spm[index] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float h_start = act ? a.h[ind] : 1.f;
+    float h_i = act && a.guess ? a.guess[index] : h_start;
+    bool guided = a.guess != nullptr;
+    float eps_last = 3.0e38f, eps_prev = 3.0e38f;
+    float h1 = 1.f / h_i, h_scan = h_i, density = 0.f;
+    int count = 0, max_h = 0, nN = 0;
+    /* as cell_box: no box for what is not finite or far outside the grid */
+    const float far = fmaxf(fmaxf(fabsf(pm.x), fabsf(pm.y)), fabsf(pm.z)) + 4.f * (fabsf(h_i) + fabsf(h_start));
+    bool redo = act && !(h_i > 0.f && h_start > 0.f && far < 1e9f * a.cells.cell_size && pm.x == pm.x &&
+                         pm.y == pm.y && pm.z == pm.z);
+    bool go = act && !redo;
+    if (!__any(go || redo)) return;
+    /* (of the step's h: the same lists with and without a guess; the cell
+     * walk's order needs the cells) */
+    const int level = S ? 0 : near_level(a.cells, 2.f * kReachGrow * h_start);
+    const Level cells = cell_level(a.cells, 0);
+    float reach = -1.f;
+    float r[NS * R], m[NS * R];
+    int cnt[P] = {};
+    int mycnt = 0, longest = 0, nrow = 0; /* own list's entries, the longest list's, its rows of GL */
+    int first[3] = {0, 0, 0};
+    /* bins: the box's shape and place modulo GL S, and the h that have it;
+     * the lane's entries in each and the most that a lane has */
+    int shape = -1;
+    float hlo = 0.f, hhi = -1.f;
+    int nb[NS] = {}, rows[NS] = {};
+    auto bin_entry = [&](int k, int e) -> int { /* place in the list of the k-th bin's e-th */
+        if constexpr (S > 0) return l.row[k][e][lane];
+        return e * GL + gl;
+    };
+    /* entries e0 .. e0 + 3 of the k-th bin: slots, records, distances */
+    auto gather = [&](int k, int e0, int n) {
+        float4 q[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = spm[e0 + e < n ? l.slot[g][bin_entry(k, e0 + e)] : 0];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float dx = q[e].x - pm.x, dy = q[e].y - pm.y, dz = q[e].z - pm.z;
+            const bool in = e0 + e < n;
+            r[k * R + e0 + e] = in ? __builtin_amdgcn_sqrtf(pair_r2(dx, dy, dz)) : 3.0e38f;
+            m[k * R + e0 + e] = in ? q[e].w : 0.f;
+        }
+    };
+    auto total = [&](const float (&v)[NS]) {
+        if constexpr (S > 0) return bins_sum<GL, S>(v);
+        return lanes_sum<GL>(v[0]);
+    };
+    while (__any(go)) {
+        const bool need = go && 2.f * h_i > reach;
+        const bool built = __any(need);
+        if (built) {
+            if (need) reach = 2.f * kReachGrow * h_i;
+#pragma unroll 1
+            for (int v = 0; v < (S ? 1 : kLevels); ++v)
+                if (__any(need && level == v))
+                    build_near_lists<GL, S, P>(cell_level(a.cells, v), spm, pm.x, pm.y, pm.z,
+                                            need && level == v ? reach : -1.f, l, cnt, first);
+            longest = 0;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                mycnt = g == p ? cnt[p] : mycnt;
+                longest = max(longest, min(cnt[p], kCap));
+            }
+            nrow = (longest + GL - 1) / GL;
+            const bool over = (need && mycnt > kCap) || redo;
+            if (over) {
+                redo = true;
+                go = false;
+                mycnt = 0;
+            }
+            if constexpr (S == 0) {
+                nb[0] = (mycnt - gl + GL - 1) / GL;
+                rows[0] = nrow;
+#pragma unroll
+                for (int e0 = 0; e0 < R; e0 += 4)
+                    if (e0 < nrow) gather(0, e0, nb[0]);
+            }
+            /* a guess so large that its list overflows: its first scan from
+             * the cells decides, and the restart has a list of its own */
+            const uint64_t ask = __ballot(over && need && guided && eps_last > 1.0e38f);
+            if (ask != 0ull) {
+                for (int p = 0; p < P; ++p) {
+                    if (((ask >> (GL * p)) & 1ull) == 0ull) continue;
+                    const float hp = lane_f(h_i, GL * p), hp1 = 1.f / hp;
+                    const float px = lane_f(pm.x, GL * p), py = lane_f(pm.y, GL * p), pz = lane_f(pm.z, GL * p);
+                    float part = 0.f;
+                    wave_near(cell_level(a.cells, __builtin_amdgcn_readlane(level, GL * p)), spm, px, py, pz, 2.f * hp,
+                              l.mark, [&](int, float4 q, bool valid, int) {
+                        const float rr = __builtin_amdgcn_sqrtf(pair_r2(q.x - px, q.y - py, q.z - pz));
+                        part += valid ? kW_tp(rr * hp1, kPi1 * hp1 * hp1 * hp1) * q.w : 0.f;
+                    });
+                    part = lanes_sum<64>(part);
+                    const float newH = 0.5f * (hp + fminf(a.res_eta * cbrtf(lane_f(pm.w, GL * p) / part), a.max_h_len));
+                    if (g == p && fabsf(newH - hp) * hp1 > kGuessTrust) {
+                        guided = redo = false;
+                        h_i = h_scan = h_start;
+                        h1 = 1.f / h_i;
+                        reach = -1.f;
+                        count++;
+                        go = count < a.max_it;
+                        density = part;
+                    }
+                }
+                continue;
+            }
+        }
+        if constexpr (S > 0) {
+            if (built || __any(go && !(h_i >= hlo && h_i <= hhi))) {
+                /* the cell walk's box for this h, and how far h may move
+                 * before one of its six faces enters another cell; the
+                 * products are within 2^-22 of cell_box's quotients */
+                const float xyz[3] = {pm.x, pm.y, pm.z};
+                int mn[3], mx[3];
+                float up = 3.0e38f, down = 3.0e38f, slack = 0.f;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float lo = (xyz[k] - 2.f * h_i) * cells.inv, hi = (xyz[k] + 2.f * h_i) * cells.inv;
+                    const float flo = floorf(lo), fhi = floorf(hi);
+                    mn[k] = (int)flo;
+                    mx[k] = (int)fhi;
+                    up = fminf(up, fminf(lo - flo, (fhi + 1.f) - hi));
+                    down = fminf(down, fminf((flo + 1.f) - lo, hi - fhi));
+                    slack = fmaxf(slack, 1e-6f * (fabsf(lo) + fabsf(hi) + 1.f));
+                }
+                up -= slack;
+                down -= slack;
+                hhi = h_i + 0.5f * cells.size * up;
+                hlo = h_i - 0.5f * cells.size * down;
+                if (!(fminf(up, down) > 0.f)) { /* on a cell's face: for this h alone */
+                    cell_box(make_float3(pm.x, pm.y, pm.z), cells.size, h_i, cells.mask + 1, mn, mx);
+                    hhi = -1.f;
+                }
+                const int ny = mx[1] - mn[1] + 1, nz = mx[2] - mn[2] + 1;
+                const int off = ((first[0] - mn[0]) * ny + (first[1] - mn[1])) * nz + (first[2] - mn[2]);
+                constexpr int kMask = GL * S - 1;
+                const int now = (ny & kMask) << 10 | (nz & kMask) << 5 | (off & kMask);
+                const bool moved = go && now != shape;
+                shape = now;
+                if (built || __any(moved)) {
+                    deal_bins<GL, S, P>(l, min(mycnt, kCap), longest, ny, nz, off, nb);
+                    bool full = false;
+#pragma unroll
+                    for (int k = 0; k < S; ++k) {
+                        rows[k] = min(wave_max(nb[k]), NearLds<GL, S, P>::kBin);
+                        full = full || nb[k] > NearLds<GL, S, P>::kBin;
+                    }
+                    /* (any lane of the group) */
+                    if (lanes_sum<GL>(full ? 1 : 0) > 0 && act) {
+                        redo = true;
+                        go = false;
+                    }
+#pragma unroll
+                    for (int k = 0; k < S; ++k)
+#pragma unroll
+                        for (int e0 = 0; e0 < R; e0 += 4)
+                            if (e0 < rows[k]) gather(k, e0, nb[k]);
+                }
+                if (!__any(go)) break;
+            }
+        }
+        const float k1 = -h1, k2 = -0.5f * h1;
+        const float fac = kPi1 * h1 * h1 * h1;
+        const bool cache = h_i < (float)max_h && nN < a.ne;
+        float sum;
+        if (__any(go && (h_i >= 1.f || max_h > 0))) {
+            /* the reference's neighbour cache may come into play (an h of 1
+             * or more): count the members, and from the cache sum only those
+             * of the last full scan */
+            const float lim = cache ? 2.f * h_scan : 3.0e38f;
+            int n = 0;
+            float part[NS];
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                part[k] = 0.f;
+                for (int e = 0; e < rows[k]; ++e) {
+                    const bool in = e < nb[k];
+                    const float4 q = spm[in ? l.slot[g][bin_entry(k, e)] : 0];
+                    const float rr = in ? __builtin_amdgcn_sqrtf(pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z)) : 3.0e38f;
+                    n += rr <= 2.f * h_i ? 1 : 0;
+                    part[k] = add_w(part[k], rr, in && rr <= lim ? q.w : 0.f, k1, k2);
+                }
+                part[k] *= fac;
+            }
+            n = lanes_sum<GL>(n);
+            if (go && !cache) nN = min(n, a.ne);
+            sum = total(part);
+        } else {
+            float part[NS];
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                part[k] = 0.f;
+#pragma unroll
+                for (int e = 0; e < R; ++e)
+                    if (e < rows[k]) part[k] = add_w(part[k], r[k * R + e], m[k * R + e], k1, k2);
+                if constexpr (S > 0)
+                    for (int e = R; e < rows[k]; ++e) {
+                        const bool in = e < nb[k];
+                        const float4 q = spm[in ? l.slot[g][bin_entry(k, e)] : 0];
+                        const float rr = __builtin_amdgcn_sqrtf(pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z));
+                        part[k] = add_w(part[k], in ? rr : 3.0e38f, in ? q.w : 0.f, k1, k2);
+                    }
+                part[k] *= fac;
+            }
+            sum = total(part);
+        }
+        float newH, eps;
+        if constexpr (S > 0) {
+            newH = fminf(a.res_eta * powf(pm.w / sum, 1.f / 3.f), a.max_h_len);
+            newH = 0.5f * (h_i + newH);
+            eps = fabsf(newH - h_i) / h_i;
+        } else {
+            newH = fminf(a.res_eta * cbrtf(pm.w / sum), a.max_h_len);
+            newH = 0.5f * (h_i + newH);
+            eps = fabsf(newH - h_i) * h1;
+        }
+        if (go) {
+            density = sum;
+            if (!cache) h_scan = h_i;
+            if (guess_rejected(guided, eps, eps_last)) {
+                /* the lists too are the plain iteration's again */
+                h_i = h_start;
+                reach = -1.f;
+                max_h = 0;
+                eps_prev = 3.0e38f;
+                count++;
+                go = count < a.max_it;
+            } else {
+                go = nr_goes_on(a.stop_rule, eps, eps_prev, a.eta);
+                eps_prev = eps;
+                if (go) {
+                    max_h = (int)fmaxf((float)max_h, h_i);
+                    h_i = newH;
+                    count++;
+                    go = count < a.max_it;
+                }
+            }
+            h1 = 1.f / h_i;
+        }
+    }
+
+    /* second pass (density.metal:146-213): over the members of the last full
+     * scan, or when they fill the reference's cache, over the box of the
+     * final h, whose density then is added to the last one (as written) or
+     * takes its place */
+    const bool fin = act && !redo;
+    const float4 vi4 = fin ? a.s_vel[index] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float hs2x4 = 4.f * h_scan * h_scan, h2x4 = 4.f * h_i * h_i, hsum = h_i + h_i;
+    int members = 0;
+    float t[5][NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        FinalSums f;
+        for (int e = 0; e < rows[k]; ++e) {
+            const bool in = fin && e < nb[k];
+            const int j = in ? l.slot[g][bin_entry(k, e)] : 0;
+            const float4 q = spm[j], vj = a.s_vel[j];
+            const float dx = q.x - pm.x, dy = q.y - pm.y, dz = q.z - pm.z;
+            const float r2 = pair_r2(dx, dy, dz);
+            const float rr = __builtin_amdgcn_sqrtf(r2);
+            members += in && !(r2 > hs2x4) ? 1 : 0;
+            if (in && !(r2 > hs2x4) && !(rr > hsum)) f.add(rr, q.w, dx, dy, dz, vj, vi4, h1);
+        }
+        t[0][k] = f.density_h;
+        t[1][k] = f.velDiv;
+        t[2][k] = f.cx;
+        t[3][k] = f.cy;
+        t[4][k] = f.cz;
+    }
+    const float density_h = total(t[0]);
+    float velDiv = total(t[1]);
+    const float cx = total(t[2]), cy = total(t[3]), cz = total(t[4]);
+    members = lanes_sum<GL>(members);
+    const bool full = members >= a.ne;
+    if (__any(full)) {
+        float part[NS];
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            part[k] = 0.f;
+            for (int e = 0; e < rows[k]; ++e)
+                if (full && e < nb[k]) {
+                    const float4 q = spm[l.slot[g][bin_entry(k, e)]];
+                    const float r2 = pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z);
+                    if (!(r2 > h2x4)) part[k] += kW_tp(__builtin_amdgcn_sqrtf(r2) * h1, kPi1 * h1 * h1 * h1) * q.w;
+                }
+        }
+        const float dpart = total(part);
+        if (full) density = (a.fix_cache ? 0.f : density) + dpart;
+        /* (only at the iteration cap do the last scan's h and the final one differ) */
+        if (full && h_scan != h_i) redo = true;
+    }
+    if ((P == 1 ? lane : gl) != 0 || !act) return;
+    if (redo) {
+        a.redo[atomicAdd(a.redo_count, 1)] = index;
+        return;
+    }
+    a.nr_iters[ind] = count;
+    velDiv = fabsf(velDiv) / density;
+    const float absCurl = sqrtf(cx * cx + cy * cy + cz * cz) / density;
+    const float fgrad = 1.f / (1.f + (h_i / (3.f * density)) * density_h);
+    const float2 pc = eos_sample(table, a.eos_res, a.u[ind], density, a.min_u, a.max_u, a.min_rho, a.max_rho);
+    const float bal = velDiv / (velDiv + absCurl + 1e-4f * (pc.y / h_i));
+    a.h[ind] = h_i;
+    a.rho[ind] = density;
+    a.f[ind] = fgrad;
+    a.P[ind] = pc.x;
+    a.c[ind] = pc.y;
+    a.B[ind] = bal;
+}
+
+/* One wave per workgroup, P particles per wave: consecutive sorted slots
+ * (LIST false, workgroups XCD-remapped) or list entries (LIST true, a
+ * persistent grid whose XCD x walks the x-th eighth of the list). */
+template <int GL, int S, bool LIST, int P = 64 / GL>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 && S ? 2 : (S ? 3 : 4)))) void k_density_lists(
+    DensityArgs a) {
+    __shared__ NearLds<GL, S, P> l;
+    const int g = P == 1 ? 0 : (int)threadIdx.x / GL;
+    if constexpr (!LIST) {
+        const int blk = xcd_block((unsigned)((a.n + P - 1) / P));
+        if (blk < 0) return;
+        const int k = blk * P + g;
+        density_chunk<GL, S, P>(a, k < a.n ? k : -1, l);
+        return;
+    }
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
+    const int total = *a.nslots;
+    const int nlog = (total + P - 1) / P;
+    const int per = (nlog + kXcds - 1) / kXcds;
+    const int xcd = (int)(blockIdx.x % kXcds), nper = (int)(gridDim.x / kXcds);
+    for (int q = (int)(blockIdx.x / kXcds); q < per; q += nper) {
+        const int lb = xcd * per + q;
+        if (lb >= nlog) break;
+        const int e = lb * P + g;
+        density_chunk<GL, S, P>(a, e < total ? a.slots[e] : -1, l);
     }
 }
 
@@ -1271,6 +1698,8 @@ Cells make_cells(const sph_ctx* ctx) {
     c.cell_se = ctx->cell_se;
     c.cell_size = ctx->prm.cell_width;
     c.mask = (1 << ctx->prm.cell_power) - 1;
+    c.block_se[0] = ctx->block_se[0];
+    c.block_se[1] = ctx->block_se[1];
     return c;
 }
 
@@ -1344,7 +1773,14 @@ int launch_density(sph_ctx* ctx) {
     a.slots = nullptr;
     a.nslots = nullptr;
     a.order = nullptr;
-    if (!a.skip_inactive && p.density_order > 0) {
+    /* From lists where the particles still lie in their cells and no option
+     * asks for the walk (its lane splits, its counts), for the numbers of
+     * lanes whose order the lists keep. */
+    const bool lists = ctx->cells_fresh && p.max_nr_iterations > 0 && (p.density_stop || p.density_eta < 1.f) &&
+                       !ctx->count_work && !p.lane_split && !p.density_flat &&
+                       (a.skip_inactive ? p.list_density_lanes == 16
+                                        : (ctx->n < p.small_n_lanes || p.density_lanes == 8));
+    if (!lists && !a.skip_inactive && p.density_order > 0) {
 #define SPH_NR_ORDER(W)                                                                                   \
     case W:                                                                                               \
         k_nr_order<W><<<(ctx->n + (W) - 1) / (W), W, 0, ctx->stream>>>(ctx->n, ctx->pairs_a, ctx->nr_iters, \
@@ -1372,6 +1808,62 @@ int launch_density(sph_ctx* ctx) {
         a.nslots = ctx->slot_count;
     }
     const int threads = 256;
+    a.redo = nullptr;
+    a.redo_count = nullptr;
+    a.clear = nullptr;
+    if (lists) {
+        /* the particles that the first launch leaves, a wave each, then what
+         * that leaves in the cell walk: three launches, the last two small or
+         * empty (near the fixed point at 1e5 the first launch's rest took the
+         * walk 275 us, the chain of its longest; a wave each, 60 us) */
+        int32_t* now = ctx->redo_count + 2 * ctx->redo_turn;
+        ctx->redo_turn ^= 1;
+        int32_t* next = ctx->redo_count + 2 * ctx->redo_turn;
+        a.redo = ctx->redo;
+        a.redo_count = now;
+        /* Near the fixed point (density_stop) the sums keep the order of the
+         * cell walk with this many lanes: h is iterated to 2.5e-6, its
+         * rounding noise shows in rho's and the pressure's last digits, and
+         * another order would change them (to 5e-5 of rho at 1e6).  The
+         * reference's rule stops 1e3 times earlier, and the even deal is 1.6x
+         * as fast: 1.36 against 2.2 ms at 1e6 for the same scans. */
+        const int order = !p.density_stop ? 0 : (a.slots ? 16 : (ctx->n < p.small_n_lanes ? 32 : 8));
+        /* 16 lanes fill the chip below 65536 particles (1 wave per SIMD at 8
+         * lanes there): 2e4 near the fixed point 0.41 ms, with 8 0.64 */
+        const int gl = ctx->n < 65536 && (order == 0 || order == 32) ? 16 : 8;
+        const unsigned waves = xcd_grid((unsigned)(((int64_t)ctx->n * gl + 63) / 64));
+        const unsigned grid = a.slots ? std::min(waves, (unsigned)kListWaves) : waves;
+        if (order == 32 && gl == 16) k_density_lists<16, 2, false><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (order == 32) k_density_lists<8, 4, false><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (order == 16) k_density_lists<8, 2, true><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (order == 8) k_density_lists<8, 1, false><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (a.slots && gl == 16) k_density_lists<16, 0, true><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (a.slots) k_density_lists<8, 0, true><<<grid, 64, 0, ctx->stream>>>(a);
+        else if (gl == 16) k_density_lists<16, 0, false><<<grid, 64, 0, ctx->stream>>>(a);
+        else k_density_lists<8, 0, false><<<grid, 64, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        a.slots = ctx->redo;
+        a.nslots = now;
+        a.redo = ctx->redo + ctx->n;
+        a.redo_count = now + 1;
+        a.clear = next;
+        const unsigned alone = std::min(xcd_grid(ctx->n), 2048u);
+        if (order == 32) k_density_lists<16, 2, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        else if (order == 16) k_density_lists<16, 1, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        else if (order == 8) k_density_lists<8, 1, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        else k_density_lists<64, 0, true><<<alone, 64, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        a.slots = a.redo;
+        a.nslots = a.redo_count;
+        next += 1;
+        a.clear = next;
+        const unsigned blocks = std::min(xcd_grid((ctx->n + 7) / 8), 512u);
+        if (order == 32) k_density_group<32, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
+        else if (order == 16) k_density_group<16, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
+        else k_density_group<8, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        return SPH_OK;
+    }
     const int flat = p.density_flat ? 1 : 0;
     const int dlanes = a.slots ? p.list_density_lanes : (ctx->n < p.small_n_lanes ? 32 : p.density_lanes);
     const int dsel = (dlanes * 2 + (p.lane_split ? 1 : 0)) * 2 + flat;
@@ -1541,7 +2033,7 @@ int launch_step(sph_ctx* ctx) {
     k_step<<<(ctx->n + threads - 1) / threads, threads, 0, ctx->stream>>>(a);
     SPH_HIP_TRY(hipGetLastError());
     ctx->dv_pending = false;
-    ctx->morton_fresh = false; /* positions and velocities moved */
+    ctx->morton_fresh = ctx->cells_fresh = false; /* positions and velocities moved */
     if (p.max_rungs > 0) {
         k_advance_time<<<1, 1, 0, ctx->stream>>>(ctx->time);
         SPH_HIP_TRY(hipGetLastError());

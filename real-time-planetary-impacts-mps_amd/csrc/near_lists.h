@@ -1,0 +1,434 @@
+/*
+ * near_lists.h -- neighbour lists of a wave's particles, built by the wave.
+ *
+ * The neighbour passes give a wave 64 / GL particles with GL lanes each.
+ * Walking the cell boxes lane by lane leaves two lanes in three idle: cells
+ * hold different numbers of particles and boxes different numbers of cells,
+ * and every walk pays for the cell table and the addresses again.  Here the
+ * wave first walks the union of its particles' boxes once, 64 candidates at
+ * a time with every lane busy, tests each candidate against the particles
+ * (their positions and radii are wave-uniform, in scalar registers) and
+ * appends the slots inside a particle's radius to that particle's list in
+ * LDS.  The passes then work on the lists, whose entries are dealt evenly to
+ * the particle's lanes.
+ */
+#ifndef NEAR_LISTS_H
+#define NEAR_LISTS_H
+
+#include "sph_internal.h"
+
+#include <type_traits>
+
+struct Cells {
+    const uint2* cell_se;
+    float cell_size;
+    int mask;
+    /* the same for blocks of 2^3 and 4^3 cells, whose slots are consecutive
+     * too (null where the grid has no such blocks) */
+    const uint2* block_se[2];
+};
+
+/* One of the cell table's levels: cells (0) or blocks of 2^3 or 4^3. */
+struct Level {
+    const uint2* se;
+    float size, inv;
+    int mask;
+};
+constexpr int kLevels = 3;
+__device__ __forceinline__ Level cell_level(const Cells& c, int level) {
+    const float size = c.cell_size * (float)(1 << level);
+    return Level{level == 0 ? c.cell_se : c.block_se[level - 1], size, 1.f / size, c.mask >> level};
+}
+/* The level to walk for a list of radius `reach`: blocks of at most about
+ * three quarters of it, so that a box holds a few hundred cells or blocks at
+ * most (a wave looks 64 up at a time) without many more candidates. */
+__device__ __forceinline__ int near_level(const Cells& c, float reach) {
+    const bool one = c.block_se[0] && reach >= 2.6f * c.cell_size;
+    return one ? (c.block_se[1] && reach >= 5.2f * c.cell_size ? 2 : 1) : 0;
+}
+
+constexpr int kPerLane = 16; /* list entries per lane */
+
+/* Data movement between lanes without LDS (DPP); lanes without a source,
+ * or outside ROWS, read `old`. */
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xF, false);
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dppf(float old, float v) {
+    return __int_as_float(dpp<CTRL, ROWS>(__float_as_int(old), __float_as_int(v)));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kHalfMirror = 0x141, kRowRor8 = 0x128;
+constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
+constexpr int kBcast15 = 0x142, kBcast31 = 0x143;
+
+/* Sum and maximum over a particle's GL lanes (8, 16, 32, 64), the same bits
+ * in each. */
+template <int GL>
+__device__ __forceinline__ float lanes_sum(float v) {
+    v += dppf<kQuadXor1>(0.f, v);
+    v += dppf<kQuadXor2>(0.f, v);
+    v += dppf<kHalfMirror>(0.f, v);
+    if constexpr (GL >= 16) v += dppf<kRowRor8>(0.f, v);
+    if constexpr (GL >= 32) v += __shfl_xor(v, 16, 64);
+    if constexpr (GL >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+template <int GL>
+__device__ __forceinline__ int lanes_sum(int v) {
+    v += dpp<kQuadXor1>(0, v);
+    v += dpp<kQuadXor2>(0, v);
+    v += dpp<kHalfMirror>(0, v);
+    if constexpr (GL >= 16) v += dpp<kRowRor8>(0, v);
+    if constexpr (GL >= 32) v += __shfl_xor(v, 16, 64);
+    if constexpr (GL >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+template <int GL>
+__device__ __forceinline__ float lanes_max(float v) {
+    v = fmaxf(v, dppf<kQuadXor1>(v, v));
+    v = fmaxf(v, dppf<kQuadXor2>(v, v));
+    v = fmaxf(v, dppf<kHalfMirror>(v, v));
+    if constexpr (GL >= 16) v = fmaxf(v, dppf<kRowRor8>(v, v));
+    if constexpr (GL >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
+    if constexpr (GL >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+/* Minimum over the wave of a value that is the same in each aligned group
+ * of 8 lanes, as a wave-uniform scalar. */
+__device__ __forceinline__ float groups_min(float v) {
+    v = fminf(v, dppf<kRowRor8>(v, v));
+    v = fminf(v, dppf<kBcast15, 0xA>(v, v));
+    v = fminf(v, dppf<kBcast31, 0xC>(v, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+/* Inclusive sum and maximum (of values >= 0) over the lanes up to this one. */
+__device__ __forceinline__ int scan_add(int v) {
+    v += dpp<kRowShr1>(0, v);
+    v += dpp<kRowShr2>(0, v);
+    v += dpp<kRowShr4>(0, v);
+    v += dpp<kRowShr8>(0, v);
+    v += dpp<kBcast15, 0xA>(0, v);
+    return v + dpp<kBcast31, 0xC>(0, v);
+}
+__device__ __forceinline__ int scan_max(int v) {
+    v = max(v, dpp<kRowShr1>(0, v));
+    v = max(v, dpp<kRowShr2>(0, v));
+    v = max(v, dpp<kRowShr4>(0, v));
+    v = max(v, dpp<kRowShr8>(0, v));
+    v = max(v, dpp<kBcast15, 0xA>(0, v));
+    return max(v, dpp<kBcast31, 0xC>(0, v));
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float lane_f(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+/* LDS accesses of one wave complete in order: this only keeps the compiler
+ * from moving them. */
+__device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+/* The lists of P particles with GL lanes each (P = 64 / GL, or 1: every group
+ * of lanes works on the same one).  S = 0: kPerLane entries per lane, and 64
+ * more places that a window may spill into.  S > 0 (the cell walk's order,
+ * deal_bins): GL S bins, S of them a lane's; a bin's first kRows entries are
+ * kept in registers; the others, up to kBin, are read again for every scan
+ * (where a box is 8 cells wide in z, say, a bin of 8 is a slab of the box and
+ * may hold a third of the list). */
+template <int GL, int S, int P, bool BINS = (S > 0)>
+struct NearLds {
+    static constexpr int kCap = GL * kPerLane, kRows = kPerLane;
+    int32_t slot[P][kCap + 64];
+    int32_t mark[64];
+};
+template <int GL, int S, int P>
+struct NearLds<GL, S, P, true> {
+    static constexpr int kCap = P == 1 ? 768 : (GL <= 8 ? 160 : 224);
+    static constexpr int kRows = (P == 1 ? 64 : (S <= 1 ? 28 : 32)) / S; /* (a multiple of 4) */
+    static constexpr int kBin = P == 1 ? 192 / S : (S <= 1 ? 64 : (S == 2 ? 40 : 24));
+    using Place = typename std::conditional<(kCap > 255), uint16_t, uint8_t>::type;
+    int32_t slot[P][kCap];
+    int32_t mark[64];
+    /* the entries' cells, 5 bits an axis, counted from the walk's first */
+    uint16_t cell[P][kCap];
+    /* the entries' bins (a byte each, in an order that turns a byte compare
+     * into a mask of entries), and each bin's entries in list order */
+    uint32_t bin[P][kCap / 4];
+    Place row[S][kBin][64];
+};
+
+/* Calls body(k, record, valid, cell) with a candidate slot, its record and
+ * its cell (counted from mn, 5 bits an axis) per lane for every particle of the cells [mn, mn + (nx, ny, nz)), 64 at a time in
+ * cell order.  `keep(ix, iy, iz)` drops cells.  The lanes take 64 cells; a
+ * prefix sum of their counts and a running maximum over marks at the cells'
+ * first candidates tell each lane which cell its candidate is of, so that
+ * the candidates of any number of cells of any size fill the wave.  The next
+ * window's records are requested before body works on this one's. */
+template <class Keep, class Body>
+__device__ __forceinline__ void wave_candidates(const Level& cells, const float4* __restrict__ spos, const int mn[3], int nx,
+                                                int ny, int nz, int32_t* mark, Keep keep, Body body) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int ncell = nx * ny * nz;
+    const float inz = 1.f / (float)nz, iny = 1.f / (float)ny;
+    for (int base = 0; base < ncell; base += 64) {
+        const int c = base + lane;
+        /* the divisions through FP32 are exact while the rounding of the
+         * quotient, 2^-22 of it, stays under half a step, 1 / (2 n) */
+        const bool small = ncell <= 1 << 18;
+        const int t = small ? (int)(((float)c + 0.5f) * inz) : c / nz, iz = c - t * nz;
+        const int ix = small ? (int)(((float)t + 0.5f) * iny) : t / ny, iy = t - ix * ny;
+        uint2 se = make_uint2(0xFFFFFFFFu, 0u);
+        if (c < ncell && keep(mn[0] + ix, mn[1] + iy, mn[2] + iz))
+            se = cells.se[dev_expand_bits((uint32_t)((mn[0] + ix) & cells.mask)) |
+                               (dev_expand_bits((uint32_t)((mn[1] + iy) & cells.mask)) << 1) |
+                               (dev_expand_bits((uint32_t)((mn[2] + iz) & cells.mask)) << 2)];
+        const int cnt = se.x == 0xFFFFFFFFu ? 0 : (int)(se.y - se.x + 1u);
+        const int incl = scan_add(cnt), excl = incl - cnt;
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        if (total == 0) continue;
+        const int shift = (int)se.x - excl; /* slot = flat index + shift of its cell's lane */
+        const int own = (ix & 31) | (iy & 31) << 5 | (iz & 31) << 10;
+        int cell;
+        auto slot_at = [&](int w) {
+            mark[lane] = 0;
+            lds_order();
+            const int at = max(excl - w, 0);
+            if (cnt > 0 && incl > w && at < 64) mark[at] = lane;
+            lds_order();
+            const int src = scan_max(mark[lane]);
+            lds_order();
+            /* the lanes past the last candidate repeat it */
+            const int f = min(w + lane, total - 1);
+            cell = __builtin_amdgcn_ds_bpermute(4 * src, own);
+            return f + __builtin_amdgcn_ds_bpermute(4 * src, shift);
+        };
+        int k = slot_at(0);
+        float4 q = spos[k];
+        for (int w = 0; w < total; w += 64) {
+            const int k0 = k, cell0 = cell;
+            const float4 q0 = q;
+            if (w + 64 < total) {
+                k = slot_at(w + 64);
+                q = spos[k];
+            }
+            body(k0, q0, w + lane < total, cell0);
+        }
+    }
+}
+
+/* The cells that hold every particle within `reach` of some particle of the
+ * lanes with `mine`, and which of them to keep. */
+struct NearBox {
+    int mn[3], nc[3];
+    float inlo[3], inhi[3], rr, cs;
+    bool whole;
+    __device__ __forceinline__ bool keep(int cx, int cy, int cz) const {
+        const float gx = fmaxf(fmaxf(inlo[0] - (float)(cx + 1) * cs, (float)cx * cs - inhi[0]), 0.f);
+        const float gy = fmaxf(fmaxf(inlo[1] - (float)(cy + 1) * cs, (float)cy * cs - inhi[1]), 0.f);
+        const float gz = fmaxf(fmaxf(inlo[2] - (float)(cz + 1) * cs, (float)cz * cs - inhi[2]), 0.f);
+        return whole || gx * gx + gy * gy + gz * gz <= rr;
+    }
+};
+__device__ __forceinline__ NearBox near_box(const Level& cells, bool mine, float x, float y, float z, float reach, float& ratio) {
+    const float big = 3.0e38f;
+    const float dim = (float)(cells.mask + 1);
+    const float rmax = -groups_min(mine ? -reach : big), rmin = groups_min(mine ? reach : big);
+    const float xyz[3] = {x, y, z};
+    NearBox b;
+    b.cs = cells.size;
+    b.rr = rmax * rmax * 1.0002f;
+    b.whole = false;
+    const float iown = 1.f / fminf(2.f * rmax * cells.inv + 2.f, dim);
+    ratio = 1.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float lo = groups_min(mine ? xyz[k] - reach : big), hi = -groups_min(mine ? -(xyz[k] + reach) : big);
+        /* the pad covers the rounding of the coordinates that the cells were
+         * assigned by; the particles lie in [inlo, inhi] */
+        const float pad = 1e-3f * cells.size + 5e-7f * (fabsf(lo) + fabsf(hi));
+        b.mn[k] = uniform((int)floorf((lo - pad) * cells.inv));
+        b.nc[k] = uniform((int)floorf((hi + pad) * cells.inv)) - b.mn[k] + 1;
+        if (b.nc[k] > cells.mask + 1) { /* the periodic grid once */
+            b.nc[k] = cells.mask + 1;
+            b.whole = true;
+        }
+        ratio *= (float)b.nc[k] * iown;
+        b.inlo[k] = lo + rmin - pad;
+        b.inhi[k] = hi - rmin + pad;
+    }
+    return b;
+}
+
+/* Calls body(k, record, valid, cell) for every candidate near one particle,
+ * at a wave-uniform (x, y, z): every particle within `reach`, and others. */
+template <class Body>
+__device__ __forceinline__ NearBox wave_near(const Level& cells, const float4* __restrict__ spos, float x, float y, float z,
+                                             float reach, int32_t* mark, Body body) {
+    float ratio;
+    const NearBox b = near_box(cells, true, x, y, z, reach, ratio);
+    wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], mark,
+                    [&](int cx, int cy, int cz) { return b.keep(cx, cy, cz); }, body);
+    return b;
+}
+
+/* A candidate's place in a list of c entries, for the lanes of m. */
+__device__ __forceinline__ int list_place(uint64_t m, int c) {
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)c));
+}
+
+/* Neighbour lists of the wave's P particles: particle p, of lane GL p, sits at
+ * (x, y, z); the slots of the candidates within `reach` go to
+ * l.slot[p][0..cnt[p]), in the order of the level's cells (cnt[p] may exceed
+ * kCap: then only the first kCap are sure to be there).  A particle with
+ * reach < 0 keeps its list and count.  A particle's list depends on its
+ * position, reach and level alone, not on the particles that share its wave.
+ * The particles are built together from the union of their boxes; when they
+ * are spread out, each from its own: a candidate of the union costs about 25
+ * instructions and 10 per particle, so that eight boxes alone cost less from
+ * a union of 2.5 of them on.  S > 0 also keeps the candidates' cells, counted
+ * from `first` (set for the lanes of the built particles); a box as wide as
+ * the periodic grid, where a cell has two places, counts as too long. */
+template <int GL, int S, int P>
+__device__ __forceinline__ void build_near_lists(const Level& cells, const float4* __restrict__ spos, float x, float y,
+                                                 float z, float reach, NearLds<GL, S, P>& l, int (&cnt)[P],
+                                                 int (&first)[3]) {
+    constexpr int kCap = NearLds<GL, S, P>::kCap;
+    const uint64_t asked = __ballot(reach >= 0.f);
+    auto append = [&](int p, bool hit, int k, int cell, int& c) {
+        const uint64_t m = __ballot(hit);
+        if constexpr (S == 0) {
+            const int at = list_place(m, min(c, kCap));
+            if (hit) l.slot[p][at] = k;
+        } else {
+            const int at = list_place(m, c);
+            if (hit && at < kCap) {
+                l.slot[p][at] = k;
+                l.cell[p][at] = (uint16_t)cell;
+            }
+        }
+        c += (int)__popcll(m);
+    };
+    float ratio;
+    const NearBox b = near_box(cells, reach >= 0.f, x, y, z, reach, ratio);
+    const float reach2 = reach * reach;
+    if ((S == 0 && P == 1) || (ratio <= 2.5f && !b.whole)) {
+        float px[P], py[P], pz[P], pr2[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            px[p] = lane_f(x, GL * p);
+            py[p] = lane_f(y, GL * p);
+            pz[p] = lane_f(z, GL * p);
+            pr2[p] = lane_f(reach2, GL * p);
+            if ((asked >> (GL * p)) & 1ull) cnt[p] = 0;
+        }
+        wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], l.mark,
+                        [&](int cx, int cy, int cz) { return b.keep(cx, cy, cz); },
+                        [&](int k, float4 q, bool valid, int cell) {
+            if (!valid) q.x = 3.0e38f;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                if (((asked >> (GL * p)) & 1ull) == 0ull) continue;
+                const float dx = q.x - px[p], dy = q.y - py[p], dz = q.z - pz[p];
+                append(p, fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= pr2[p], k, cell, cnt[p]);
+            }
+        });
+        if (S > 0 && reach >= 0.f)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) first[j] = b.mn[j];
+    } else {
+        for (int p = 0; p < P; ++p) {
+            if (((asked >> (GL * p)) & 1ull) == 0ull) continue;
+            const float px = lane_f(x, GL * p), py = lane_f(y, GL * p), pz = lane_f(z, GL * p);
+            const float rp = lane_f(reach, GL * p), rp2 = lane_f(reach2, GL * p);
+            int c = 0;
+            const NearBox own = wave_near(cells, spos, px, py, pz, rp, l.mark, [&](int k, float4 q, bool valid, int cell) {
+                const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
+                append(p, valid && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= rp2, k, cell, c);
+            });
+            if (S > 0 && own.whole) c = kCap + 1;
+#pragma unroll
+            for (int j = 0; j < P; ++j) cnt[j] = j == p ? c : cnt[j];
+            if (S > 0 && (P == 1 || (int)(threadIdx.x & 63) / GL == p))
+#pragma unroll
+                for (int j = 0; j < 3; ++j) first[j] = own.mn[j];
+        }
+    }
+    lds_order();
+}
+
+/* The order of the sums of the cell walk with G = GL S lanes per particle:
+ * there lane b sums the candidates of cells b, b + G, ... of the particle's
+ * box in order, and the lanes' sums are added in a fixed tree.  This deals a
+ * list's entries to the same G bins, bins b, b + GL, ... to the particle's
+ * lane b, so that the same terms are added in the same order, bit for bit.
+ * The bin of an entry is its cell's position in the box, modulo G, which
+ * changes with the box: `ny`, `nz` are the box's cells in y and z and `off`
+ * the position, in it, of the cell that the list's cells are counted from.
+ * (An entry outside the box is beyond 2h: it adds 0 to whichever bin.)
+ * n[k] = entries of the lane's k-th bin (it may exceed kBin). */
+template <int GL, int S, int P>
+__device__ __forceinline__ void deal_bins(NearLds<GL, S, P>& l, int have, int longest, int ny, int nz, int off, int (&n)[S]) {
+    constexpr uint32_t kNone = 0x40u, kMask = GL * S - 1;
+    static_assert(GL * S <= 32, "cells are kept modulo 32");
+    const int lane = (int)(threadIdx.x & 63), gl = lane % GL, g = P == 1 ? 0 : lane / GL;
+    uint8_t* bytes = reinterpret_cast<uint8_t*>(l.bin[g]);
+    /* entry 32 W + p in byte p / 8 of word 8 W + p % 8 */
+    auto byte_at = [](int i) { return (i & ~31) + ((i & 7) << 2) + ((i >> 3) & 3); };
+    const int words = (longest + 31) / 32;
+    const int sx = (ny * nz) & kMask, sy = nz & kMask;
+#pragma unroll 4
+    for (int i = gl; i < words * 32; i += GL) {
+        uint32_t bin = kNone;
+        if (i < have) {
+            const int c = l.cell[g][i];
+            bin = (uint32_t)(__mul24(c & 31, sx) + __mul24((c >> 5) & 31, sy) + (c >> 10) + off) & kMask;
+        }
+        bytes[byte_at(i)] = (uint8_t)bin;
+    }
+    lds_order();
+    uint32_t c = 0; /* entries of the lane's bins so far, a byte each */
+    constexpr uint32_t kLane = (kNone | (GL - 1)) * 0x01010101u;
+    const uint32_t mine = (uint32_t)gl * 0x01010101u;
+    for (int w = 0; w < words; ++w) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t v = (l.bin[g][8 * w + k] ^ mine) & kLane; /* zero byte: a bin of this lane's */
+            m |= (~(v + 0x7F7F7F7Fu) & 0x80808080u) >> (7 - k);
+        }
+        while (__any(m != 0u)) {
+            if (m != 0u) {
+                const int i = 32 * w + __ffs((int)m) - 1;
+                m &= m - 1u;
+                const int k = S > 1 ? (int)(bytes[byte_at(i)] / GL) : 0;
+                const int at = (int)((c >> (8 * k)) & 255u);
+                if (at < NearLds<GL, S, P>::kBin) l.row[k][at][lane] = (typename NearLds<GL, S, P>::Place)i;
+                if (at < 255) c += 1u << (8 * k);
+            }
+        }
+    }
+    lds_order();
+#pragma unroll
+    for (int k = 0; k < S; ++k) n[k] = (int)((c >> (8 * k)) & 255u);
+}
+
+/* The cell walk's tree over its G = GL S lanes (distances G/2, ..., 1); no
+ * product is drawn into its additions. */
+template <int GL, int S>
+__device__ __forceinline__ float bins_sum(const float (&v)[S]) {
+#pragma clang fp contract(off)
+    float t = S == 4 ? (v[0] + v[2 % S]) + (v[1 % S] + v[3 % S]) : (S == 2 ? v[0] + v[1 % S] : v[0]);
+    if constexpr (GL == 16) t += dppf<kRowRor8>(0.f, t);
+    /* lanes 4 apart within 8: up for the low half, down for the high */
+    const float x = dppf<0x104>(0.f, t), y = dppf<0x114>(0.f, t); /* row_shl 4, row_shr 4 */
+    t += (threadIdx.x & 4) ? y : x;
+    t += dppf<kQuadXor2>(0.f, t);
+    return t + dppf<kQuadXor1>(0.f, t);
+}
+/* Maximum over the wave of a value >= 0. */
+__device__ __forceinline__ int wave_max(int v) { return __builtin_amdgcn_readlane(scan_max(v), 63); }
+
+#endif

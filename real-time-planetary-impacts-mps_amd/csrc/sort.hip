@@ -191,26 +191,43 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint2* __restrict__ 
     }
 }
 
+/* The slot ranges of blocks of 2^3 and 4^3 cells (null: none): a block's
+ * cells share their key's high bits, so its particles are consecutive too. */
+struct Blocks {
+    uint2* se[2];
+};
+
 /* Resets the cells that the previous sort occupied (sparse form of
  * `initialise`, sort.metal:131-138). */
-__global__ void k_cells_reset(const uint2* __restrict__ prev, int n, uint2* __restrict__ cell_se) {
+__global__ void k_cells_reset(const uint2* __restrict__ prev, int n, uint2* __restrict__ cell_se, Blocks blocks) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t key = prev[i].x;
-    if (i == 0 || prev[i - 1].x != key) cell_se[key] = make_uint2(0xFFFFFFFFu, 0u);
+    const uint32_t key = prev[i].x, changed = i == 0 ? 0xFFFFFFFFu : prev[i - 1].x ^ key;
+    if (changed) cell_se[key] = make_uint2(0xFFFFFFFFu, 0u);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if (blocks.se[k] && changed >> (3 * (k + 1))) blocks.se[k][key >> (3 * (k + 1))] = make_uint2(0xFFFFFFFFu, 0u);
 }
 
 /* findCellPositions (sort.metal:140-148) from run boundaries, fused with the
  * gather of the Morton-ordered copies used by the neighbour passes. */
-__global__ void k_cells_gather(const uint2* __restrict__ sorted, int n, uint2* __restrict__ cell_se,
+__global__ void k_cells_gather(const uint2* __restrict__ sorted, int n, uint2* __restrict__ cell_se, Blocks blocks,
                                const float4* __restrict__ pos, const float4* __restrict__ vel,
                                const float* __restrict__ m, float4* __restrict__ s_posm, float4* __restrict__ s_vel) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint2 pr = sorted[i];
     const uint32_t key = pr.x;
-    if (i == 0 || sorted[i - 1].x != key) cell_se[key].x = (uint32_t)i;
-    if (i == n - 1 || sorted[i + 1].x != key) cell_se[key].y = (uint32_t)i;
+    const uint32_t begins = i == 0 ? 0xFFFFFFFFu : sorted[i - 1].x ^ key;
+    const uint32_t ends = i == n - 1 ? 0xFFFFFFFFu : sorted[i + 1].x ^ key;
+    if (begins) cell_se[key].x = (uint32_t)i;
+    if (ends) cell_se[key].y = (uint32_t)i;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int bits = 3 * (k + 1);
+        if (blocks.se[k] && begins >> bits) blocks.se[k][key >> bits].x = (uint32_t)i;
+        if (blocks.se[k] && ends >> bits) blocks.se[k][key >> bits].y = (uint32_t)i;
+    }
     const uint32_t j = pr.y;
     const float4 p = pos[j];
     const float4 v = vel[j];
@@ -229,6 +246,12 @@ int launch_fill_cells(sph_ctx* ctx) {
     const int threads = 256;
     k_fill_cells<<<(ctx->ncells + threads - 1) / threads, threads, 0, ctx->stream>>>(ctx->cell_se, ctx->ncells);
     SPH_HIP_TRY(hipGetLastError());
+    for (int k = 0; k < 2; ++k) {
+        if (!ctx->block_se[k]) continue;
+        const int count = ctx->ncells >> (3 * (k + 1));
+        k_fill_cells<<<(count + threads - 1) / threads, threads, 0, ctx->stream>>>(ctx->block_se[k], count);
+        SPH_HIP_TRY(hipGetLastError());
+    }
     return SPH_OK;
 }
 
@@ -268,8 +291,9 @@ int launch_sort(sph_ctx* ctx) {
     const int threads = 256;
     const int blocks = (n + threads - 1) / threads;
     hipStream_t s = ctx->stream;
+    const Blocks tables{{ctx->block_se[0], ctx->block_se[1]}};
     if (ctx->have_prev) {
-        k_cells_reset<<<blocks, threads, 0, s>>>(ctx->prev_keys_src, n, ctx->cell_se);
+        k_cells_reset<<<blocks, threads, 0, s>>>(ctx->prev_keys_src, n, ctx->cell_se, tables);
         SPH_HIP_TRY(hipGetLastError());
     }
     uint2* bufs[2] = {ctx->pairs_a, ctx->pairs_b};
@@ -291,7 +315,7 @@ int launch_sort(sph_ctx* ctx) {
         cur ^= 1;
     }
     uint2* sorted = bufs[cur];
-    k_cells_gather<<<blocks, threads, 0, s>>>(sorted, n, ctx->cell_se, ctx->pos, ctx->vel, ctx->m, ctx->s_posm,
+    k_cells_gather<<<blocks, threads, 0, s>>>(sorted, n, ctx->cell_se, tables, ctx->pos, ctx->vel, ctx->m, ctx->s_posm,
                                               ctx->s_vel);
     SPH_HIP_TRY(hipGetLastError());
     /* keep the sorted array where the next sort will not overwrite it before

@@ -9,6 +9,7 @@
  *     mat, next_active, nr_iters            int32 x n;  active uint8 x n
  *   cells: pairs_a / pairs_b  uint2 x n (sorted (key, index), ping-pong)
  *          cell_se            uint2 x C (first slot, last slot), 128 MiB at C = 2^24
+ *          block_se           uint2 x C / 8, C / 64: the same for blocks of cells
  *   Morton-ordered copies written once per pass and read by every
  *   neighbour candidate (slot k = k-th sorted particle):
  *          s_posm  float4 (x, y, z, m)        -- written after the sort
@@ -155,6 +156,8 @@ struct sph_ctx {
     uint2* prev_keys_src = nullptr;               /* sorted pairs of the previous sort (for the sparse reset) */
     bool have_prev = false;
     uint2* cell_se = nullptr;
+    /* the same for blocks of 2^3 and 4^3 cells (null below cell_power 2, 3) */
+    uint2* block_se[2] = {nullptr, nullptr};
     uint32_t* tile_hist = nullptr; /* 256 x ntiles, digit-major */
     uint32_t* digit_total = nullptr; /* 256: pairs per digit of the current pass */
     int ntiles = 0;
@@ -163,6 +166,10 @@ struct sph_ctx {
      * particles' positions, masses and velocities (set by a sort, cleared by a
      * step or an upload of those fields) */
     bool morton_fresh = false;
+    /* the cells still hold the particles by their positions (set by a sort,
+     * cleared by a step or an upload of positions): a particle's candidates
+     * are then all within its radius, whatever box of cells they come from */
+    bool cells_fresh = false;
     /* the density pass fills density_work (and runs without its neighbour
      * lists) only while this is set: sph_set_work_counters */
     bool count_work = false;
@@ -219,6 +226,11 @@ struct sph_ctx {
     int32_t* slot_list = nullptr;   /* sorted slots of the active particles (README rule) */
     int32_t* slot_count = nullptr;  /* their number (device) */
     bool slot_list_valid = false;   /* cleared by a sort and by a gravity pass */
+    /* slots the list-built density pass's first and second launch leave to
+     * the next (n each), and their counts: two pairs in turn, each cleared by
+     * the pass before */
+    int32_t *redo = nullptr, *redo_count = nullptr;
+    int redo_turn = 0;
     sph_mlp* learned = nullptr;     /* not owned */
     sph_samples* dump = nullptr;    /* not owned */
 };
@@ -285,6 +297,8 @@ constexpr int kDownBlocks = 2048;
 /* the largest grid of the hydro passes' persistent launches over the active
  * particles' slots (README rule) */
 constexpr int kListBlocks = 2048;
+/* the largest grid, in workgroups of one wave, of the list-built passes' */
+constexpr int kListWaves = 8192;
 inline unsigned xcd_grid(unsigned blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
 __device__ __forceinline__ int xcd_block(unsigned blocks) {
     const unsigned per = (blocks + kXcds - 1) / kXcds;
