@@ -171,8 +171,8 @@ struct DensityArgs {
     /* every slot: the order in which the groups take them (k_nr_order), or
      * null for slot order */
     const int32_t* order;
-    /* k_density_lists: the slots it leaves to a grouped launch over `redo`
-     * and their count; that launch clears the count the next pass uses */
+    /* k_density_lists: the slots it leaves to the next launch over `redo` and
+     * their count; a count that this launch clears for a later one */
     int32_t* redo;
     int32_t* redo_count;
     int32_t* clear;
@@ -945,7 +945,7 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                     const float px = lane_f(pm.x, GL * p), py = lane_f(pm.y, GL * p), pz = lane_f(pm.z, GL * p);
                     float part = 0.f;
                     wave_near(cell_level(a.cells, __builtin_amdgcn_readlane(level, GL * p)), spm, px, py, pz, 2.f * hp,
-                              l.mark, [&](int, float4 q, bool valid, int) {
+                              l.walk, [&](int, float4 q, bool valid, int) {
                         const float rr = __builtin_amdgcn_sqrtf(pair_r2(q.x - px, q.y - py, q.z - pz));
                         part += valid ? kW_tp(rr * hp1, kPi1 * hp1 * hp1 * hp1) * q.w : 0.f;
                     });
@@ -1175,6 +1175,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 && S 
     DensityArgs a) {
     __shared__ NearLds<GL, S, P> l;
     const int g = P == 1 ? 0 : (int)threadIdx.x / GL;
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if constexpr (!LIST) {
         const int blk = xcd_block((unsigned)((a.n + P - 1) / P));
         if (blk < 0) return;
@@ -1182,7 +1183,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 && S 
         density_chunk<GL, S, P>(a, k < a.n ? k : -1, l);
         return;
     }
-    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     const int total = *a.nslots;
     const int nlog = (total + P - 1) / P;
     const int per = (nlog + kXcds - 1) / kXcds;
@@ -1348,6 +1348,11 @@ struct AccelArgs {
      * on the device; null: every slot */
     const int32_t* slots;
     const int32_t* nslots;
+    /* k_accel_lists: the slots it leaves to the next launch over `redo` and
+     * their count; a count that this launch clears for a later one */
+    int32_t* redo;
+    int32_t* redo_count;
+    int32_t* clear;
 };
 
 /* accelerations.metal:130-136: the step goal 2 CFL Gamma h / v_sig; with
@@ -1364,6 +1369,17 @@ __device__ __forceinline__ int wave_min(int v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
     return v;
+}
+
+/* time[1] = min(time[1], v) for a wave.  Atomics on one address take their
+ * turn, about 50 ns each (a wave of 8 particles, at 1e6: 7.4 ms, and 1.0 with
+ * the question): a wave asks first whether its step is the smaller one, and
+ * once the smallest is there no wave's is.  (A value read too early is too
+ * large, and costs an atomic.) */
+__device__ __forceinline__ void min_step(int32_t* time, int v) {
+    const int wmin = wave_min(v);
+    if ((threadIdx.x & 63) == 0 && wmin < __hip_atomic_load(&time[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(&time[1], wmin);
 }
 
 /* accelerations.metal:12-141 */
@@ -1467,6 +1483,7 @@ __device__ __forceinline__ int accel_particle(const AccelArgs& a, int index) {
 /* 8 waves per SIMD (64 VGPRs, no spills) with the candidate prefetch */
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_acceleration(AccelArgs a) {
     int integerDt = 0x7FFFFFFF;
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if (!a.slots) {
         const int blk = xcd_block((a.n + 255) / 256);
         if (blk < 0) return;
@@ -1483,8 +1500,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
             integerDt = min(integerDt, accel_particle(a, e < total ? a.slots[e] : -1));
         }
     }
-    const int wmin = wave_min(integerDt);
-    if ((threadIdx.x & 63) == 0 && wmin != 0x7FFFFFFF) atomicMin(&a.time[1], wmin);
+    min_step(a.time, integerDt);
 }
 
 /* accelerations.metal:12-141 with G lanes per particle, the box split as
@@ -1598,6 +1614,7 @@ __global__ __launch_bounds__(256) void k_acceleration_group(AccelArgs a) {
     constexpr int PPB = 256 / G;
     const int lane = threadIdx.x % G, g = (int)threadIdx.x / G;
     int integerDt = 0x7FFFFFFF;
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if constexpr (!LIST) {
         const int blk = xcd_block((a.n + PPB - 1) / PPB);
         if (blk < 0) return;
@@ -1614,8 +1631,219 @@ __global__ __launch_bounds__(256) void k_acceleration_group(AccelArgs a) {
             integerDt = min(integerDt, accel_group_particle<G, SPLIT>(a, e < total ? a.slots[e] : -1, lane));
         }
     }
-    const int wmin = wave_min(integerDt);
-    if ((threadIdx.x & 63) == 0 && wmin != 0x7FFFFFFF) atomicMin(&a.time[1], wmin);
+    min_step(a.time, integerDt);
+}
+
+/* The pair term of accel_particle with its roundings (the fused
+ * multiply-adds that the compiler forms there, written out). */
+struct PairTerm {
+    float x, y, z, u; /* -(...) of dv, and du's, to be multiplied by m and added in order */
+    float vgi;        /* dh/dt's, to be multiplied by mr */
+    float m, mr;
+};
+__device__ __forceinline__ PairTerm pair_term(const AccelArgs& a, float4 xi4, float4 vi4, float4 hi, float hi1, float faci,
+                                              float4 xj4, float4 vj4, float4 hj, float& v_sigi) {
+    const float dx = xi4.x - xj4.x, dy = xi4.y - xj4.y, dz = xi4.z - xj4.z;
+    const float r = __builtin_amdgcn_sqrtf(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
+    const float r1 = __builtin_amdgcn_rcpf(r), hj1 = __builtin_amdgcn_rcpf(xj4.w);
+    const float vx = vi4.x - vj4.x, vy = vi4.y - vj4.y, vz = vi4.z - vj4.z;
+    const float rho_ij = 0.5f * (hi.z + hj.z);
+    const float v_dot_r = fmaf(vz, dz, fmaf(vx, dx, vy * dy));
+    const float mu = v_dot_r < 0.f ? v_dot_r * r1 : 0.f;
+    const float v_sig = fmaf(-3.f, mu, hi.w + hj.w);
+    v_sigi = fmaxf(v_sig, v_sigi);
+    const float nu = -0.5f * a.alpha * (0.5f * (vi4.w + vj4.w)) * mu * v_sig * __builtin_amdgcn_rcpf(rho_ij);
+    const float rx = dx * r1, ry = dy * r1, rz = dz * r1;
+    const float ai = fmaxf(fmaf(-hi1, r, 2.f), 0.f), bi = fmaxf(fmaf(-hi1, r, 1.f), 0.f);
+    const float aj = fmaxf(fmaf(-hj1, r, 2.f), 0.f), bj = fmaxf(fmaf(-hj1, r, 1.f), 0.f);
+    const float gi = faci * fmaf(bi, 3.f * bi, -(ai * (0.75f * ai)));
+    const float gj = kPi1 * hj1 * hj1 * hj1 * hj1 * fmaf(bj, 3.f * bj, -(aj * (0.75f * aj)));
+    const float gix = rx * gi, giy = ry * gi, giz = rz * gi;
+    const float gjx = rx * gj, gjy = ry * gj, gjz = rz * gj;
+    const float gmx = 0.5f * fmaf(rx, gj, gix), gmy = 0.5f * fmaf(ry, gj, giy), gmz = 0.5f * fmaf(rz, gj, giz);
+    const float vgi = fmaf(vz, giz, fmaf(vx, gix, vy * giy)), vgm = fmaf(vz, gmz, fmaf(vx, gmx, vy * gmy));
+    PairTerm t;
+    t.x = -fmaf(gmx, nu, fmaf(hi.y, gix, hj.y * gjx));
+    t.y = -fmaf(gmy, nu, fmaf(hi.y, giy, hj.y * gjy));
+    t.z = -fmaf(gmz, nu, fmaf(hi.y, giz, hj.y * gjz));
+    t.u = fmaf(hi.y, vgi, 0.5f * nu * vgm);
+    t.vgi = vgi;
+    t.m = hj.x;
+    t.mr = hj.x * __builtin_amdgcn_rcpf(hj.z);
+    return t;
+}
+
+/* The pair lists of P particles and a tile of their pairs' terms; a
+ * particle's part is padded by 8 words so that the groups' reads of one term
+ * fall on different banks. */
+template <int GL, bool SERIAL, int P>
+struct AccelLds {
+    static constexpr int kLanes = 64 / P, kTile = P == 1 ? 1 : 2;
+    NearLds<GL, 1, P, !SERIAL || P == 1, false> l;
+    union {
+        float term[P][kTile * kLanes * 8 + 8];
+        WalkLds walk;
+    };
+};
+
+/* accelerations.metal:12-141 for the wave's P particles (64 / P lanes each),
+ * from lists of their pairs: the candidates of the cell boxes that pass the
+ * pair test, in the cell walk's order.  The lanes evaluate the list's terms,
+ * a tile at a time, into LDS, and the tile is then added up in the order of
+ * the walk: by one lane per sum (SERIAL, accel_particle's order), or by the
+ * lane of each of GL bins and the tree over them (accel_group_particle<GL>'s,
+ * bins as deal_bins deals them).  The sums have the walk's bits.
+ *
+ * In the walk a lane in two holds a candidate that fails the test while the
+ * others evaluate the 90 instructions of a pair.  Here they fill the wave, and
+ * the pass is bound by VALU issue: 4000 instructions per wave of 8 particles
+ * at 1e6, half of them the test of the 13 windows of candidates.  The pass,
+ * walk -> lists (with min_step's question), ms: 0.49 -> 0.19 at 2e4, 0.93 ->
+ * 0.31 at 1e5, 0.77 -> 0.37 at 3e5, 1.68 -> 1.04 at 1e6, 5.4 -> 4.1 at 4e6.
+ *
+ * Particles with more pairs than a list or a bin holds are left to `redo`. */
+template <int GL, bool SERIAL, int P>
+__device__ __forceinline__ int accel_chunk(const AccelArgs& a, int index, AccelLds<GL, SERIAL, P>& s) {
+    constexpr int kLanes = AccelLds<GL, SERIAL, P>::kLanes, kTile = AccelLds<GL, SERIAL, P>::kTile;
+    constexpr int kCap = decltype(s.l)::kCap;
+    const int lane = (int)(threadIdx.x & 63), pl = lane % kLanes, g = lane / kLanes, gl = lane % GL;
+    const bool on = index >= 0;
+    const uint32_t ind = on ? a.sorted[index].y : 0u;
+    const bool act = on && a.active[ind];
+    if (!__any(act)) return 0x7FFFFFFF;
+    const float4 xi4 = act ? a.s_posh[index] : make_float4(0.f, 0.f, 0.f, 1.f);
+    int mn[3] = {0, 0, 0}, mx[3] = {-1, -1, -1};
+    if (act)
+        cell_box(make_float3(xi4.x, xi4.y, xi4.z), a.cells.cell_size, fminf(xi4.w, a.max_h_len), a.cells.mask + 1, mn, mx);
+    int cnt[P], ny, nz, off;
+    build_pair_lists<kLanes, P>(cell_level(a.cells, 0), a.s_posh, xi4, mn, mx, s.l, s.walk, cnt, ny, nz, off);
+    int mycnt = 0;
+    int longest = 0;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        mycnt = g == p ? cnt[p] : mycnt;
+        longest = max(longest, min(cnt[p], kCap));
+    }
+    bool redo = act && mycnt > kCap;
+    mycnt = redo ? 0 : mycnt;
+    int nb[1] = {0};
+    if constexpr (!SERIAL) {
+        deal_bins<GL, 1, P>(s.l, mycnt, longest, ny, nz, off, nb);
+        if (lanes_sum<GL>(nb[0] > decltype(s.l)::kBin ? 1 : 0) > 0 && act) {
+            redo = true;
+            mycnt = 0;
+            nb[0] = 0;
+        }
+    }
+    const float4 vi4 = act ? a.s_velb[index] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 hyd = act ? a.s_hyd[index] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float h_i = xi4.w, hi1 = 1.f / h_i, faci = kPi1 * hi1 * hi1 * hi1 * hi1;
+    float v_sigi = 1e-12f;
+    float sum[5] = {0.f, 0.f, 0.f, 0.f, 0.f}; /* SERIAL: lane q's in sum[0], q = 0 .. 4 */
+    int at = 0;                               /* bins: entries added */
+    float* term = s.term[g];
+    for (int base = 0; base < longest; base += kTile * kLanes) {
+        float4 xj[kTile], vj[kTile], hj[kTile];
+#pragma unroll
+        for (int e = 0; e < kTile; ++e) {
+            const int i = base + e * kLanes + pl, k = i < mycnt ? s.l.slot[g][i] : 0;
+            xj[e] = a.s_posh[k];
+            vj[e] = a.s_velb[k];
+            hj[e] = a.s_hyd[k];
+        }
+#pragma unroll
+        for (int e = 0; e < kTile; ++e) {
+            /* past the end: terms whose products are -0, which changes no sum */
+            PairTerm t{-0.f, -0.f, -0.f, -0.f, -0.f, 0.f, 0.f};
+            if (base + e * kLanes + pl < mycnt) t = pair_term(a, xi4, vi4, hyd, hi1, faci, xj[e], vj[e], hj[e], v_sigi);
+            float4* w = reinterpret_cast<float4*>(term + (e * kLanes + pl) * 8);
+            w[0] = make_float4(t.x, t.y, t.z, t.u);
+            w[1] = make_float4(t.vgi, t.m, t.mr, 0.f);
+        }
+        lds_order();
+        if constexpr (SERIAL) {
+            const int q = min(pl, 4), mq = q == 4 ? 6 : 5;
+#pragma unroll 8
+            for (int e = 0; e < kTile * kLanes; ++e) sum[0] = fmaf(term[e * 8 + mq], term[e * 8 + q], sum[0]);
+        } else {
+            const int end = base + kTile * kLanes;
+            for (;;) {
+                int i = 0x7FFFFFFF;
+                if (at < nb[0]) i = s.l.row[0][at][lane];
+                const bool in = i < end;
+                if (!__any(in)) break;
+                if (in) {
+                    const float4* w = reinterpret_cast<const float4*>(term + (i - base) * 8);
+                    const float4 t = w[0], m = w[1];
+                    sum[0] = fmaf(m.y, t.x, sum[0]);
+                    sum[1] = fmaf(m.y, t.y, sum[1]);
+                    sum[2] = fmaf(m.y, t.z, sum[2]);
+                    sum[3] = fmaf(m.y, t.w, sum[3]);
+                    sum[4] = fmaf(m.z, m.x, sum[4]);
+                    ++at;
+                }
+            }
+        }
+        lds_order();
+    }
+    v_sigi = lanes_max<kLanes>(v_sigi);
+    if constexpr (SERIAL) {
+        const float mine = sum[0];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) sum[q] = __shfl(mine, (lane & ~(kLanes - 1)) + q, 64);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            const float v[1] = {sum[q]};
+            sum[q] = bins_sum<GL, 1>(v);
+        }
+    }
+    if (pl != 0 || !act) return 0x7FFFFFFF;
+    if (redo) {
+        a.redo[atomicAdd(a.redo_count, 1)] = index;
+        return 0x7FFFFFFF;
+    }
+    a.dv[ind] = make_float4(sum[0], sum[1], sum[2], 0.f);
+    a.du[ind] = sum[3];
+    a.dhdt[ind] = sum[4];
+    const float goaldt = step_goal(a, h_i, v_sigi, sum[4]);
+    int r = 0;
+    float dtCandidate = a.dt0;
+    while (dtCandidate > goaldt && r < a.r_max) {
+        dtCandidate *= 0.5f;
+        r++;
+    }
+    const int integerDt = (int)ceilf(a.dtmin * dtCandidate);
+    a.next_active[ind] = a.time[0] + integerDt;
+    return integerDt;
+}
+
+/* One wave per workgroup, P particles per wave, over every slot or a list as
+ * k_density_lists. */
+template <int GL, bool SERIAL, bool LIST, int P = 64 / GL>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 ? 2 : 4))) void k_accel_lists(AccelArgs a) {
+    __shared__ AccelLds<GL, SERIAL, P> s;
+    const int g = (int)threadIdx.x / (64 / P);
+    int integerDt = 0x7FFFFFFF;
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
+    if constexpr (!LIST) {
+        const int blk = xcd_block((unsigned)((a.n + P - 1) / P));
+        if (blk < 0) return;
+        const int k = blk * P + g;
+        integerDt = accel_chunk<GL, SERIAL, P>(a, k < a.n ? k : -1, s);
+    } else {
+        const int total = *a.nslots;
+        const int nlog = (total + P - 1) / P;
+        const int per = (nlog + kXcds - 1) / kXcds;
+        const int xcd = (int)(blockIdx.x % kXcds), nper = (int)(gridDim.x / kXcds);
+        for (int q = (int)(blockIdx.x / kXcds); q < per; q += nper) {
+            const int lb = xcd * per + q;
+            if (lb >= nlog) break;
+            const int e = lb * P + g;
+            integerDt = min(integerDt, accel_chunk<GL, SERIAL, P>(a, e < total ? a.slots[e] : -1, s));
+        }
+    }
+    min_step(a.time, integerDt);
 }
 
 struct StepArgs {
@@ -1816,11 +2044,9 @@ int launch_density(sph_ctx* ctx) {
          * that leaves in the cell walk: three launches, the last two small or
          * empty (near the fixed point at 1e5 the first launch's rest took the
          * walk 275 us, the chain of its longest; a wave each, 60 us) */
-        int32_t* now = ctx->redo_count + 2 * ctx->redo_turn;
-        ctx->redo_turn ^= 1;
-        int32_t* next = ctx->redo_count + 2 * ctx->redo_turn;
         a.redo = ctx->redo;
-        a.redo_count = now;
+        a.redo_count = ctx->redo_count;
+        a.clear = ctx->redo_count + 1;
         /* Near the fixed point (density_stop) the sums keep the order of the
          * cell walk with this many lanes: h is iterated to 2.5e-6, its
          * rounding noise shows in rho's and the pressure's last digits, and
@@ -1843,10 +2069,10 @@ int launch_density(sph_ctx* ctx) {
         else k_density_lists<8, 0, false><<<grid, 64, 0, ctx->stream>>>(a);
         SPH_HIP_TRY(hipGetLastError());
         a.slots = ctx->redo;
-        a.nslots = now;
+        a.nslots = ctx->redo_count;
         a.redo = ctx->redo + ctx->n;
-        a.redo_count = now + 1;
-        a.clear = next;
+        a.redo_count = ctx->redo_count + 1;
+        a.clear = nullptr;
         const unsigned alone = std::min(xcd_grid(ctx->n), 2048u);
         if (order == 32) k_density_lists<16, 2, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
         else if (order == 16) k_density_lists<16, 1, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
@@ -1855,8 +2081,7 @@ int launch_density(sph_ctx* ctx) {
         SPH_HIP_TRY(hipGetLastError());
         a.slots = a.redo;
         a.nslots = a.redo_count;
-        next += 1;
-        a.clear = next;
+        a.clear = ctx->redo_count;
         const unsigned blocks = std::min(xcd_grid((ctx->n + 7) / 8), 512u);
         if (order == 32) k_density_group<32, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
         else if (order == 16) k_density_group<16, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
@@ -1966,6 +2191,36 @@ int launch_acceleration(sph_ctx* ctx) {
     SPH_HIP_TRY(hipGetLastError());
     const int alanes = a.slots ? p.list_accel_lanes
                                : (ctx->n < p.small_n_lanes ? (ctx->n < 65536 ? 16 : 8) : p.accel_lanes);
+    a.redo = nullptr;
+    a.redo_count = nullptr;
+    a.clear = nullptr;
+    if (!p.lane_split && (a.slots ? alanes == 16 : (alanes == 0 || alanes == 8 || alanes == 16))) {
+        /* from lists, summed in the order of the walk with that many lanes;
+         * what the first launch leaves a wave each, then the walk */
+        a.redo = ctx->redo;
+        a.redo_count = ctx->redo_count;
+        a.clear = ctx->redo_count + 1;
+        const int gl = alanes == 16 ? 16 : 8;
+        const unsigned waves = xcd_grid((unsigned)(((int64_t)ctx->n * gl + 63) / 64));
+        if (a.slots) k_accel_lists<16, false, true><<<std::min(waves, (unsigned)kListWaves), 64, 0, ctx->stream>>>(a);
+        else if (alanes == 16) k_accel_lists<16, false, false><<<waves, 64, 0, ctx->stream>>>(a);
+        else if (alanes == 8) k_accel_lists<8, false, false><<<waves, 64, 0, ctx->stream>>>(a);
+        else k_accel_lists<8, true, false><<<waves, 64, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        a.slots = ctx->redo;
+        a.nslots = ctx->redo_count;
+        a.redo = ctx->redo + ctx->n;
+        a.redo_count = ctx->redo_count + 1;
+        a.clear = nullptr;
+        const unsigned alone = std::min(xcd_grid(ctx->n), 2048u);
+        if (alanes == 16) k_accel_lists<16, false, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        else if (alanes == 8) k_accel_lists<8, false, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        else k_accel_lists<8, true, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        a.slots = a.redo;
+        a.nslots = a.redo_count;
+        a.clear = ctx->redo_count;
+    }
     const int asel = alanes * 2 + (p.lane_split ? 1 : 0);
     /* over a slot list the grid is persistent: at most kListBlocks workgroups */
 #define SPH_ACC(G, S)                                                                                    \
@@ -1976,12 +2231,15 @@ int launch_acceleration(sph_ctx* ctx) {
     else                                                                                                 \
         k_acceleration_group<G, S, false>                                                                \
             <<<xcd_grid((ctx->n + (256 / (G)) - 1) / (256 / (G))), threads, 0, ctx->stream>>>(a)
+#define SPH_ACC_REST(G)                                                                                  \
+    k_acceleration_group<G, 0, true>                                                                     \
+        <<<std::min(xcd_grid((ctx->n + (256 / (G)) - 1) / (256 / (G))), (unsigned)kListBlocks), threads, 0, ctx->stream>>>(a)
     switch (asel) {
         case 4: SPH_ACC(2, 0); break;
         case 8: SPH_ACC(4, 0); break;
-        case 16: SPH_ACC(8, 0); break;
+        case 16: SPH_ACC_REST(8); break; /* (the lists' rest) */
         case 17: SPH_ACC(8, 1); break;
-        case 32: SPH_ACC(16, 0); break;
+        case 32: SPH_ACC_REST(16); break;
         case 33: SPH_ACC(16, 1); break;
         case 64: SPH_ACC(32, 0); break;
         case 65: SPH_ACC(32, 1); break;
@@ -1994,6 +2252,7 @@ int launch_acceleration(sph_ctx* ctx) {
         }
     }
 #undef SPH_ACC
+#undef SPH_ACC_REST
     SPH_HIP_TRY(hipGetLastError());
     ctx->dv_pending = true;
     return SPH_OK;

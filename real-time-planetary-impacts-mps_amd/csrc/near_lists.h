@@ -103,6 +103,12 @@ __device__ __forceinline__ float groups_min(float v) {
     v = fminf(v, dppf<kBcast31, 0xC>(v, v));
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
+__device__ __forceinline__ int groups_min_i(int v) {
+    v = min(v, dpp<kRowRor8>(v, v));
+    v = min(v, dpp<kBcast15, 0xA>(v, v));
+    v = min(v, dpp<kBcast31, 0xC>(v, v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
 /* Inclusive sum and maximum (of values >= 0) over the lanes up to this one. */
 __device__ __forceinline__ int scan_add(int v) {
     v += dpp<kRowShr1>(0, v);
@@ -131,6 +137,13 @@ __device__ __forceinline__ void lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
+/* The walk's: marks of a window, and a queue of cells that hold particles. */
+struct WalkLds {
+    int32_t mark[64];
+    uint2 se[128];
+    int32_t tag[128];
+};
+
 /* The lists of P particles with GL lanes each (P = 64 / GL, or 1: every group
  * of lanes works on the same one).  S = 0: kPerLane entries per lane, and 64
  * more places that a window may spill into.  S > 0 (the cell walk's order,
@@ -138,83 +151,135 @@ __device__ __forceinline__ void lds_order() {
  * kept in registers; the others, up to kBin, are read again for every scan
  * (where a box is 8 cells wide in z, say, a bin of 8 is a slab of the box and
  * may hold a third of the list). */
-template <int GL, int S, int P, bool BINS = (S > 0)>
+struct NoWalk {};
+template <int GL, int S, int P, bool BINS = (S > 0), bool WALK = true>
 struct NearLds {
     static constexpr int kCap = GL * kPerLane, kRows = kPerLane;
     int32_t slot[P][kCap + 64];
-    int32_t mark[64];
+    typename std::conditional<WALK, WalkLds, NoWalk>::type walk;
 };
-template <int GL, int S, int P>
-struct NearLds<GL, S, P, true> {
+template <int GL, int S, int P, bool WALK>
+struct NearLds<GL, S, P, true, WALK> {
     static constexpr int kCap = P == 1 ? 768 : (GL <= 8 ? 160 : 224);
     static constexpr int kRows = (P == 1 ? 64 : (S <= 1 ? 28 : 32)) / S; /* (a multiple of 4) */
     static constexpr int kBin = P == 1 ? 192 / S : (S <= 1 ? 64 : (S == 2 ? 40 : 24));
     using Place = typename std::conditional<(kCap > 255), uint16_t, uint8_t>::type;
     int32_t slot[P][kCap];
-    int32_t mark[64];
     /* the entries' cells, 5 bits an axis, counted from the walk's first */
     uint16_t cell[P][kCap];
-    /* the entries' bins (a byte each, in an order that turns a byte compare
-     * into a mask of entries), and each bin's entries in list order */
-    uint32_t bin[P][kCap / 4];
-    Place row[S][kBin][64];
+    union {
+        struct {
+            /* the entries' bins (a byte each, in an order that turns a byte
+             * compare into a mask of entries), and each bin's entries in list
+             * order */
+            uint32_t bin[P][kCap / 4];
+            Place row[S][kBin][64];
+        };
+        typename std::conditional<WALK, WalkLds, NoWalk>::type walk; /* while the lists are built */
+    };
 };
 
-/* Calls body(k, record, valid, cell) with a candidate slot, its record and
- * its cell (counted from mn, 5 bits an axis) per lane for every particle of the cells [mn, mn + (nx, ny, nz)), 64 at a time in
- * cell order.  `keep(ix, iy, iz)` drops cells.  The lanes take 64 cells; a
- * prefix sum of their counts and a running maximum over marks at the cells'
- * first candidates tell each lane which cell its candidate is of, so that
- * the candidates of any number of cells of any size fill the wave.  The next
- * window's records are requested before body works on this one's. */
-template <class Keep, class Body>
+/* A candidate's place in a list of c entries, for the lanes of m. */
+__device__ __forceinline__ int list_place(uint64_t m, int c) {
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)c));
+}
+
+/* A cell's place counted from a walk's first, 5 bits an axis. */
+__device__ __forceinline__ int cell_place(int ix, int iy, int iz) { return (ix & 31) | (iy & 31) << 5 | (iz & 31) << 10; }
+
+/* From this many cells on the walk queues those with particles.  The queue
+ * costs a trip through LDS per 64 cells; without it every 64 cells take a
+ * window of their own, however few particles they hold.  The density and
+ * acceleration pass with and without, ms, at 2e4 (80 look-ups of 64 cells per
+ * wave) 0.30 + 0.20 and 0.41 + 0.30, at 1e5 (24) 0.82 + 0.30 and 0.87 + 0.35, at
+ * 1e6 (4) 6.19 + 1.07 and 5.80 + 1.01. */
+constexpr int kQueueFrom = 512;
+
+/* Calls body(k, record, valid, tag) with a candidate slot, its record and
+ * its cell's tag per lane for every particle of nx x ny x nz cells from mn on,
+ * 64 at a time in cell order.  tag_of(ix, iy, iz), counted from mn, is a
+ * cell's tag, or negative to drop it.  The lanes look 64 cells up and a queue
+ * keeps those that hold particles; for 64 of them a prefix sum of their counts
+ * and a running maximum over marks at their first candidates tell each lane
+ * which cell its candidate is of, so that the candidates of any number of
+ * cells of any size fill the wave.  The next window's records are requested
+ * before body works on this one's. */
+template <class Tag, class Body>
 __device__ __forceinline__ void wave_candidates(const Level& cells, const float4* __restrict__ spos, const int mn[3], int nx,
-                                                int ny, int nz, int32_t* mark, Keep keep, Body body) {
+                                                int ny, int nz, WalkLds& lds, Tag tag_of, Body body) {
     const int lane = (int)(threadIdx.x & 63);
     const int ncell = nx * ny * nz;
     const float inz = 1.f / (float)nz, iny = 1.f / (float)ny;
-    for (int base = 0; base < ncell; base += 64) {
-        const int c = base + lane;
+    const bool small = ncell <= 1 << 18;
+    int next_tag = -1;
+    uint2 next_se = make_uint2(0xFFFFFFFFu, 0u);
+    auto look_up = [&](int c) {
         /* the divisions through FP32 are exact while the rounding of the
          * quotient, 2^-22 of it, stays under half a step, 1 / (2 n) */
-        const bool small = ncell <= 1 << 18;
         const int t = small ? (int)(((float)c + 0.5f) * inz) : c / nz, iz = c - t * nz;
         const int ix = small ? (int)(((float)t + 0.5f) * iny) : t / ny, iy = t - ix * ny;
-        uint2 se = make_uint2(0xFFFFFFFFu, 0u);
-        if (c < ncell && keep(mn[0] + ix, mn[1] + iy, mn[2] + iz))
-            se = cells.se[dev_expand_bits((uint32_t)((mn[0] + ix) & cells.mask)) |
+        next_se = make_uint2(0xFFFFFFFFu, 0u);
+        next_tag = c < ncell ? tag_of(ix, iy, iz) : -1;
+        if (next_tag >= 0)
+            next_se = cells.se[dev_expand_bits((uint32_t)((mn[0] + ix) & cells.mask)) |
                                (dev_expand_bits((uint32_t)((mn[1] + iy) & cells.mask)) << 1) |
                                (dev_expand_bits((uint32_t)((mn[2] + iz) & cells.mask)) << 2)];
-        const int cnt = se.x == 0xFFFFFFFFu ? 0 : (int)(se.y - se.x + 1u);
+    };
+    const bool queue = ncell > kQueueFrom;
+    int head = 0, queued = 0; /* the queue's first cell and its length */
+    look_up(lane);
+    for (int base = 0; base < ncell || queued > 0; base += 64) {
+        /* the next cells' ranges are requested before these are used */
+        uint2 se = next_se;
+        int own = next_tag;
+        if (base + 64 < ncell) look_up(base + 64 + lane);
+        bool some = se.x != 0xFFFFFFFFu && base < ncell;
+        if (queue) {
+            const uint64_t m = __ballot(some);
+            if (some) {
+                const int at = (head + queued + list_place(m, 0)) & 127;
+                lds.se[at] = se;
+                lds.tag[at] = own;
+            }
+            queued += (int)__popcll(m);
+            if (queued < 64 && base + 64 < ncell) continue;
+            lds_order();
+            const int at = (head + lane) & 127;
+            some = lane < queued;
+            se = lds.se[at];
+            own = lds.tag[at];
+            head += 64;
+            queued = max(queued - 64, 0);
+        }
+        const int cnt = some ? (int)(se.y - se.x + 1u) : 0;
         const int incl = scan_add(cnt), excl = incl - cnt;
         const int total = __builtin_amdgcn_readlane(incl, 63);
         if (total == 0) continue;
         const int shift = (int)se.x - excl; /* slot = flat index + shift of its cell's lane */
-        const int own = (ix & 31) | (iy & 31) << 5 | (iz & 31) << 10;
-        int cell;
+        int tag;
         auto slot_at = [&](int w) {
-            mark[lane] = 0;
+            lds.mark[lane] = 0;
             lds_order();
             const int at = max(excl - w, 0);
-            if (cnt > 0 && incl > w && at < 64) mark[at] = lane;
+            if (cnt > 0 && incl > w && at < 64) lds.mark[at] = lane;
             lds_order();
-            const int src = scan_max(mark[lane]);
+            const int src = scan_max(lds.mark[lane]);
             lds_order();
             /* the lanes past the last candidate repeat it */
             const int f = min(w + lane, total - 1);
-            cell = __builtin_amdgcn_ds_bpermute(4 * src, own);
+            tag = __builtin_amdgcn_ds_bpermute(4 * src, own);
             return f + __builtin_amdgcn_ds_bpermute(4 * src, shift);
         };
         int k = slot_at(0);
         float4 q = spos[k];
         for (int w = 0; w < total; w += 64) {
-            const int k0 = k, cell0 = cell;
+            const int k0 = k, tag0 = tag;
             const float4 q0 = q;
             if (w + 64 < total) {
                 k = slot_at(w + 64);
                 q = spos[k];
             }
-            body(k0, q0, w + lane < total, cell0);
+            body(k0, q0, w + lane < total, tag0);
         }
     }
 }
@@ -225,11 +290,12 @@ struct NearBox {
     int mn[3], nc[3];
     float inlo[3], inhi[3], rr, cs;
     bool whole;
-    __device__ __forceinline__ bool keep(int cx, int cy, int cz) const {
+    __device__ __forceinline__ int tag(int ix, int iy, int iz) const {
+        const int cx = mn[0] + ix, cy = mn[1] + iy, cz = mn[2] + iz;
         const float gx = fmaxf(fmaxf(inlo[0] - (float)(cx + 1) * cs, (float)cx * cs - inhi[0]), 0.f);
         const float gy = fmaxf(fmaxf(inlo[1] - (float)(cy + 1) * cs, (float)cy * cs - inhi[1]), 0.f);
         const float gz = fmaxf(fmaxf(inlo[2] - (float)(cz + 1) * cs, (float)cz * cs - inhi[2]), 0.f);
-        return whole || gx * gx + gy * gy + gz * gz <= rr;
+        return whole || gx * gx + gy * gy + gz * gz <= rr ? cell_place(ix, iy, iz) : -1;
     }
 };
 __device__ __forceinline__ NearBox near_box(const Level& cells, bool mine, float x, float y, float z, float reach, float& ratio) {
@@ -262,21 +328,16 @@ __device__ __forceinline__ NearBox near_box(const Level& cells, bool mine, float
     return b;
 }
 
-/* Calls body(k, record, valid, cell) for every candidate near one particle,
+/* Calls body(k, record, valid, place) for every candidate near one particle,
  * at a wave-uniform (x, y, z): every particle within `reach`, and others. */
 template <class Body>
 __device__ __forceinline__ NearBox wave_near(const Level& cells, const float4* __restrict__ spos, float x, float y, float z,
-                                             float reach, int32_t* mark, Body body) {
+                                             float reach, WalkLds& lds, Body body) {
     float ratio;
     const NearBox b = near_box(cells, true, x, y, z, reach, ratio);
-    wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], mark,
-                    [&](int cx, int cy, int cz) { return b.keep(cx, cy, cz); }, body);
+    wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], lds,
+                    [&](int ix, int iy, int iz) { return b.tag(ix, iy, iz); }, body);
     return b;
-}
-
-/* A candidate's place in a list of c entries, for the lanes of m. */
-__device__ __forceinline__ int list_place(uint64_t m, int c) {
-    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)c));
 }
 
 /* Neighbour lists of the wave's P particles: particle p, of lane GL p, sits at
@@ -324,8 +385,8 @@ __device__ __forceinline__ void build_near_lists(const Level& cells, const float
             pr2[p] = lane_f(reach2, GL * p);
             if ((asked >> (GL * p)) & 1ull) cnt[p] = 0;
         }
-        wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], l.mark,
-                        [&](int cx, int cy, int cz) { return b.keep(cx, cy, cz); },
+        wave_candidates(cells, spos, b.mn, b.nc[0], b.nc[1], b.nc[2], l.walk,
+                        [&](int ix, int iy, int iz) { return b.tag(ix, iy, iz); },
                         [&](int k, float4 q, bool valid, int cell) {
             if (!valid) q.x = 3.0e38f;
 #pragma unroll
@@ -344,7 +405,7 @@ __device__ __forceinline__ void build_near_lists(const Level& cells, const float
             const float px = lane_f(x, GL * p), py = lane_f(y, GL * p), pz = lane_f(z, GL * p);
             const float rp = lane_f(reach, GL * p), rp2 = lane_f(reach2, GL * p);
             int c = 0;
-            const NearBox own = wave_near(cells, spos, px, py, pz, rp, l.mark, [&](int k, float4 q, bool valid, int cell) {
+            const NearBox own = wave_near(cells, spos, px, py, pz, rp, l.walk, [&](int k, float4 q, bool valid, int cell) {
                 const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
                 append(p, valid && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= rp2, k, cell, c);
             });
@@ -354,6 +415,110 @@ __device__ __forceinline__ void build_near_lists(const Level& cells, const float
             if (S > 0 && (P == 1 || (int)(threadIdx.x & 63) / GL == p))
 #pragma unroll
                 for (int j = 0; j < 3; ++j) first[j] = own.mn[j];
+        }
+    }
+    lds_order();
+}
+
+/* Lists of the pairs of the acceleration pass for the wave's P particles of
+ * LANES lanes each: the candidates of the particle's own cell box [mn, mx]
+ * (empty: none) within 2 h of either side, in the order of the cells.  The
+ * union of the boxes is walked once where it is less than 2.5 of the largest
+ * (and no wider than the periodic grid), each box alone otherwise.  ny, nz and
+ * off are those of deal_bins for the lane's particle. */
+template <int LANES, int P, class Lds>
+__device__ __forceinline__ void build_pair_lists(const Level& cells, const float4* __restrict__ s_posh, float4 xi,
+                                                 const int mn[3], const int mx[3], Lds& l, WalkLds& walk, int (&cnt)[P], int& ny,
+                                                 int& nz, int& off) {
+    constexpr int kCap = Lds::kCap;
+    constexpr bool kSpill = sizeof(l.slot[0]) / sizeof(l.slot[0][0]) > kCap;
+    int nc[3];
+    float own = 1.f, ratio = 1.f;
+    int umn[3], unc[3];
+    const bool some = mx[0] >= mn[0] && mx[1] >= mn[1] && mx[2] >= mn[2];
+    bool wide = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        nc[k] = mx[k] - mn[k] + 1;
+        own *= (float)nc[k];
+        umn[k] = groups_min_i(some ? mn[k] : 0x7FFFFFFF);
+        unc[k] = -groups_min_i(some ? -mx[k] : 0x7FFFFFFF) - umn[k] + 1;
+        wide = wide || unc[k] > cells.mask + 1;
+        ratio *= (float)unc[k];
+    }
+    const uint64_t asked = __ballot(some);
+#pragma unroll
+    for (int p = 0; p < P; ++p) cnt[p] = 0;
+    ny = nc[1];
+    nz = nc[2];
+    off = 0;
+    if (asked == 0ull) return;
+    const float hi2x4 = xi.w * xi.w * 4.f;
+    auto append = [&](int p, bool hit, int k, int place, int& c) {
+        const uint64_t m = __ballot(hit);
+        const int at = list_place(m, kSpill ? min(c, kCap) : c);
+        if (hit && (kSpill || at < kCap)) {
+            l.slot[p][at] = k;
+            if constexpr (!kSpill) l.cell[p][at] = (uint16_t)place;
+        }
+        c += (int)__popcll(m);
+    };
+    /* the walk's own test, form for form */
+    auto skip = [](float4 q, float px, float py, float pz, float pi2x4, float qj2x4) {
+        const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+        const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+        return (r2 > pi2x4 && r2 > qj2x4) || r2 < 1e-12f;
+    };
+    if (P == 1 || (!wide && ratio <= -2.5f * groups_min(some ? -own : 0.f))) {
+        float px[P], py[P], pz[P], ph[P];
+        int pmn[P][3], pnc[P][3];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            px[p] = lane_f(xi.x, LANES * p);
+            py[p] = lane_f(xi.y, LANES * p);
+            pz[p] = lane_f(xi.z, LANES * p);
+            ph[p] = lane_f(hi2x4, LANES * p);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                pmn[p][k] = __builtin_amdgcn_readlane(mn[k], LANES * p) - umn[k];
+                pnc[p][k] = __builtin_amdgcn_readlane(some ? nc[k] : 0, LANES * p);
+            }
+        }
+        wave_candidates(cells, s_posh, umn, unc[0], unc[1], unc[2], walk,
+                        [&](int ix, int iy, int iz) {
+            int m = 0;
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+                m |= ((unsigned)(ix - pmn[p][0]) < (unsigned)pnc[p][0] && (unsigned)(iy - pmn[p][1]) < (unsigned)pnc[p][1] &&
+                      (unsigned)(iz - pmn[p][2]) < (unsigned)pnc[p][2]) ? 1 << p : 0;
+            return m == 0 ? -1 : m << 15 | cell_place(ix, iy, iz);
+        }, [&](int k, float4 q, bool valid, int tag) {
+            const float qj2x4 = q.w * q.w * 4.f;
+            if (!valid) tag = 0;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const bool in = (tag & (1 << (15 + p))) != 0;
+                if (__any(in)) append(p, in && !skip(q, px[p], py[p], pz[p], ph[p], qj2x4), k, tag & 0x7FFF, cnt[p]);
+            }
+        });
+        off = ((umn[0] - mn[0]) * ny + (umn[1] - mn[1])) * nz + (umn[2] - mn[2]);
+    } else {
+        for (int p = 0; p < P; ++p) {
+            if (((asked >> (LANES * p)) & 1ull) == 0ull) continue;
+            const float px = lane_f(xi.x, LANES * p), py = lane_f(xi.y, LANES * p), pz = lane_f(xi.z, LANES * p);
+            const float ph = lane_f(hi2x4, LANES * p);
+            int m[3], n[3], c = 0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                m[k] = __builtin_amdgcn_readlane(mn[k], LANES * p);
+                n[k] = __builtin_amdgcn_readlane(nc[k], LANES * p);
+            }
+            wave_candidates(cells, s_posh, m, n[0], n[1], n[2], walk, cell_place,
+                            [&](int k, float4 q, bool valid, int tag) {
+                append(p, valid && !skip(q, px, py, pz, ph, q.w * q.w * 4.f), k, tag, c);
+            });
+#pragma unroll
+            for (int j = 0; j < P; ++j) cnt[j] = j == p ? c : cnt[j];
         }
     }
     lds_order();
@@ -369,8 +534,8 @@ __device__ __forceinline__ void build_near_lists(const Level& cells, const float
  * the position, in it, of the cell that the list's cells are counted from.
  * (An entry outside the box is beyond 2h: it adds 0 to whichever bin.)
  * n[k] = entries of the lane's k-th bin (it may exceed kBin). */
-template <int GL, int S, int P>
-__device__ __forceinline__ void deal_bins(NearLds<GL, S, P>& l, int have, int longest, int ny, int nz, int off, int (&n)[S]) {
+template <int GL, int S, int P, class Lds>
+__device__ __forceinline__ void deal_bins(Lds& l, int have, int longest, int ny, int nz, int off, int (&n)[S]) {
     constexpr uint32_t kNone = 0x40u, kMask = GL * S - 1;
     static_assert(GL * S <= 32, "cells are kept modulo 32");
     const int lane = (int)(threadIdx.x & 63), gl = lane % GL, g = P == 1 ? 0 : lane / GL;
@@ -405,7 +570,7 @@ __device__ __forceinline__ void deal_bins(NearLds<GL, S, P>& l, int have, int lo
                 m &= m - 1u;
                 const int k = S > 1 ? (int)(bytes[byte_at(i)] / GL) : 0;
                 const int at = (int)((c >> (8 * k)) & 255u);
-                if (at < NearLds<GL, S, P>::kBin) l.row[k][at][lane] = (typename NearLds<GL, S, P>::Place)i;
+                if (at < Lds::kBin) l.row[k][at][lane] = (typename Lds::Place)i;
                 if (at < 255) c += 1u << (8 * k);
             }
         }

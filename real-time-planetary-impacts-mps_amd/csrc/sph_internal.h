@@ -226,11 +226,10 @@ struct sph_ctx {
     int32_t* slot_list = nullptr;   /* sorted slots of the active particles (README rule) */
     int32_t* slot_count = nullptr;  /* their number (device) */
     bool slot_list_valid = false;   /* cleared by a sort and by a gravity pass */
-    /* slots the list-built density pass's first and second launch leave to
-     * the next (n each), and their counts: two pairs in turn, each cleared by
-     * the pass before */
+    /* slots that the first and the second launch of a list-built pass leave
+     * to the next (n each), and their counts: a pass's first launch clears the
+     * second count, its last the first one */
     int32_t *redo = nullptr, *redo_count = nullptr;
-    int redo_turn = 0;
     sph_mlp* learned = nullptr;     /* not owned */
     sph_samples* dump = nullptr;    /* not owned */
 };
