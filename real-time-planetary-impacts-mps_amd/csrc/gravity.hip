@@ -234,23 +234,39 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e) {
     e = (a - (s - bb)) + (b - bb);
 }
 
+/* The up pass is a chain of levels, each as long as one node's loads one after
+ * the other: a leaf's members (a batch) and a branch's children are requested
+ * together.  The 8 levels, us, one by one and together: 115 and 63 at 2e4, 225 and
+ * 135 at 1e6; precision form at 2e5 186 and 106. */
+constexpr int kBatch = 8;
+
 /* P2M.metal:12-107 */
 template <bool PREC>
 __device__ void p2m(const UpArgs& a, int id, int np, int tp) {
     const int32_t* pl = a.t.octree + tp + 2;
     const int gt = a.time[0];
+    /* the first kBatch members' records are requested together and kept */
+    int mp[kBatch], mna[kBatch];
+    float4 mx4[kBatch];
+    float mgn[kBatch];
+    const int nb = min(np, kBatch);
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) mp[k] = pl[min(k, np - 1)];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+        mx4[k] = a.pos[mp[k]];
+        mna[k] = a.next_active[mp[k]];
+        mgn[k] = a.gravnorm[mp[k]];
+    }
     float M = 0.f, px = 0.f, py = 0.f, pz = 0.f;
     float minGrav = FLT_MAX;
     bool act = false;
     float mnx = FLT_MAX, mny = FLT_MAX, mnz = FLT_MAX, mxx = -FLT_MAX, mxy = -FLT_MAX, mxz = -FLT_MAX;
     /* precision form: sum m (x - x_0) instead of m x, x_0 = first particle */
-    const float4 x0 = PREC ? a.pos[pl[0]] : make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int k = 0; k < np; ++k) {
-        const int p = pl[k];
-        const float4 xa = a.pos[p];
+    const float4 x0 = PREC ? mx4[0] : make_float4(0.f, 0.f, 0.f, 0.f);
+    auto mass_of = [&](float4 xa, int na, float gn) {
         const float pm = xa.w; /* the position record carries the mass */
         const float4 x = make_float4(xa.x - x0.x, xa.y - x0.y, xa.z - x0.z, 0.f);
-        const int na = a.next_active[p];
         const bool isActive = a.readme_rule ? (na <= gt) : (gt <= na);
         act = act || isActive;
         mxx = fmaxf(mxx, xa.x); mxy = fmaxf(mxy, xa.y); mxz = fmaxf(mxz, xa.z);
@@ -259,9 +275,19 @@ __device__ void p2m(const UpArgs& a, int id, int np, int tp) {
         px += x.x * pm;
         py += x.y * pm;
         pz += x.z * pm;
-        if (isActive) minGrav = fminf(minGrav, a.gravnorm[p]);
+        if (isActive) minGrav = fminf(minGrav, gn);
+    };
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+        if (k < nb) mass_of(mx4[k], mna[k], mgn[k]);
+    for (int k = kBatch; k < np; ++k) {
+        const int p = pl[k];
+        mass_of(a.pos[p], a.next_active[p], a.gravnorm[p]);
     }
-    for (int k = 0; k < np; ++k) a.active[pl[k]] = act ? 1 : 0;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+        if (k < nb) a.active[mp[k]] = act ? 1 : 0;
+    for (int k = kBatch; k < np; ++k) a.active[pl[k]] = act ? 1 : 0;
     /* precision form: the centre as x_0 + (offset) in two parts, the second
      * the residual of the first's rounding, so that offsets from the centre
      * keep the bits an FP32 absolute position (|x| ~ 20, ulp ~ 2e-6) drops */
@@ -278,9 +304,7 @@ __device__ void p2m(const UpArgs& a, int id, int np, int tp) {
     }
     float X = 0.f, Y = 0.f, Z = 0.f, XX = 0.f, XY = 0.f, XZ = 0.f, YY = 0.f, YZ = 0.f, ZZ = 0.f;
     float o[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < np; ++k) {
-        const int p = pl[k];
-        const float4 x = a.pos[p];
+    auto moments_of = [&](float4 x) {
         const float pm = x.w;
         /* x - px is exact where x and px are within a factor 2 of each other
          * (every leaf away from the coordinate planes) */
@@ -306,7 +330,11 @@ __device__ void p2m(const UpArgs& a, int id, int np, int tp) {
             o[8] -= pm * ry * rz * rz;
             o[9] -= pm * rz * rz * rz;
         }
-    }
+    };
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+        if (k < nb) moments_of(mx4[k]);
+    for (int k = kBatch; k < np; ++k) moments_of(a.pos[pl[k]]);
     XX *= 0.5f;
     YY *= 0.5f;
     ZZ *= 0.5f;
@@ -335,40 +363,60 @@ __device__ void p2m(const UpArgs& a, int id, int np, int tp) {
 /* M2M.metal:75-160 with transformMultipole (M2M.metal:12-73) */
 template <bool PREC>
 __device__ void m2m(const UpArgs& a, int id, int tp) {
-    const int32_t* ch = a.t.child + 8 * id;
+    int ch[8];
+    {
+        const int4* c4 = reinterpret_cast<const int4*>(a.t.child + 8 * id);
+        const int4 lo = c4[0], hi = c4[1];
+        ch[0] = lo.x; ch[1] = lo.y; ch[2] = lo.z; ch[3] = lo.w;
+        ch[4] = hi.x; ch[5] = hi.y; ch[6] = hi.z; ch[7] = hi.w;
+    }
+    /* (an empty child's place: the node's own records, not used) */
+    float4 far0[8], far1[8], far2[8], aux0[8], aux1[8], low[8];
+    float dipz[8];
+    int npart[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int k = ch[c] < 0 ? id : ch[c];
+        far0[c] = a.t.far[3 * k];
+        far1[c] = a.t.far[3 * k + 1];
+        far2[c] = a.t.far[3 * k + 2];
+        aux0[c] = a.t.aux[3 * k];
+        aux1[c] = a.t.aux[3 * k + 1];
+        dipz[c] = a.fix_zz ? 0.f : a.t.aux[3 * k + 2].z;
+        npart[c] = a.t.info[k].x;
+        if constexpr (PREC) low[c] = a.t.clo[k];
+    }
     float minGrav = FLT_MAX, mass = 0.f, px = 0.f, py = 0.f, pz = 0.f;
     bool act = false, allLeaves = true;
     float mnx = FLT_MAX, mny = FLT_MAX, mnz = FLT_MAX, mxx = -FLT_MAX, mxy = -FLT_MAX, mxz = -FLT_MAX;
     /* precision form: centre of mass relative to the first child's */
     float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (PREC)
-        for (int c = 0; c < 8; ++c)
-            if (ch[c] >= 0) {
-                r0 = a.t.far[3 * ch[c]];
-                break;
-            }
+#pragma unroll
+        for (int c = 7; c >= 0; --c)
+            if (ch[c] >= 0) r0 = far0[c];
+#pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const int cid = ch[c];
-        if (cid < 0) continue;
-        float4 f0 = a.t.far[3 * cid];
-        const float4 f1 = a.t.far[3 * cid + 1];
+        if (ch[c] < 0) continue;
+        float4 f0 = far0[c];
+        const float4 f1 = far1[c];
         f0.x -= r0.x;
         f0.y -= r0.y;
         f0.z -= r0.z;
         if constexpr (PREC) { /* the child's centre in two parts */
-            const float4 cl = a.t.clo[cid];
+            const float4 cl = low[c];
             f0.x += cl.x;
             f0.y += cl.y;
             f0.z += cl.z;
         }
-        const float4 x0 = a.t.aux[3 * cid], x1 = a.t.aux[3 * cid + 1];
+        const float4 x0 = aux0[c], x1 = aux1[c];
         minGrav = fminf(x0.w, minGrav);
         mass += f1.x;
         px += f0.x * f1.x;
         py += f0.y * f1.x;
         pz += f0.z * f1.x;
         act = act || (x1.w != 0.f);
-        if (allLeaves && a.t.info[cid].x == 0) allLeaves = false;
+        if (allLeaves && npart[c] == 0) allLeaves = false;
         mxx = fmaxf(mxx, x1.x); mxy = fmaxf(mxy, x1.y); mxz = fmaxf(mxz, x1.z);
         mnx = fminf(mnx, x0.x); mny = fminf(mny, x0.y); mnz = fminf(mnz, x0.z);
     }
@@ -386,20 +434,21 @@ __device__ void m2m(const UpArgs& a, int id, int tp) {
     }
     float M = 0.f, XX = 0.f, XY = 0.f, XZ = 0.f, YY = 0.f, YZ = 0.f, ZZ = 0.f;
     float o[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
     for (int c = 0; c < 8; ++c) {
         const int cid = ch[c];
         if (cid < 0) continue;
-        const float4 f0 = a.t.far[3 * cid], f1 = a.t.far[3 * cid + 1], f2 = a.t.far[3 * cid + 2];
+        const float4 f0 = far0[c], f1 = far1[c], f2 = far2[c];
         float rx = px - f0.x, ry = py - f0.y, rz = pz - f0.z;
         if constexpr (PREC) {
-            const float4 cl = a.t.clo[cid];
+            const float4 cl = low[c];
             rx += clx - cl.x;
             ry += cly - cl.y;
             rz += clz - cl.z;
         }
         const float cM = f1.x;
         /* as written the ZZ shift uses the child's dipole Z (M2M.metal:29) */
-        const float zzw = a.fix_zz ? cM : a.t.aux[3 * cid + 2].z;
+        const float zzw = a.fix_zz ? cM : dipz[c];
         M += cM;
         XX += f1.y + 0.5f * rx * rx * cM;
         XY += f1.z + rx * ry * cM;
@@ -422,7 +471,7 @@ __device__ void m2m(const UpArgs& a, int id, int tp) {
             o[1] += q0.y + ry * cxx + rx * cxy + 0.5f * rx * rx * ry * cM;
             o[0] += q0.x + rx * cxx + sixth * rx * rx * rx * cM;
         }
-        if (allLeaves && act && a.t.aux[3 * cid + 1].w == 0.f) {
+        if (allLeaves && act && aux1[c].w == 0.f) {
             /* leaf-sync activation (M2M.metal:145-154); as written the end of
              * the particle range starts from the parent's record */
             a.t.aux[3 * cid + 1].w = 1.f;
@@ -442,7 +491,7 @@ __device__ void m2m(const UpArgs& a, int id, int tp) {
 }
 
 template <bool PREC>
-__global__ __launch_bounds__(256) void k_up(UpArgs a) {
+__global__ __launch_bounds__(64) void k_up(UpArgs a) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= a.count || a.flags[0] != 0u) return;
     const int id = a.level_id[s];
@@ -458,11 +507,16 @@ __global__ __launch_bounds__(256) void k_up(UpArgs a) {
      * child starts where the previous child's subtree ends. */
     int end = id + 1;
     bool ordered = true;
+    int cid[8], cend[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) cid[c] = a.t.child[8 * id + c];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) cend[c] = a.t.sub_end[cid[c] < 0 ? id : cid[c]];
+#pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const int cid = a.t.child[8 * id + c];
-        if (cid < 0) continue;
-        ordered = ordered && cid == end;
-        end = a.t.sub_end[cid];
+        if (cid[c] < 0) continue;
+        ordered = ordered && cid[c] == end;
+        end = cend[c];
     }
     a.t.sub_end[id] = end;
     if (!ordered && a.need_preorder) a.flags[0] = 2u;
@@ -1681,7 +1735,7 @@ int launch_gravity_up(sph_ctx* ctx) {
     a.prec = ctx->prm.precision ? 1 : 0;
     a.order = ctx->prm.expansion_order == 3 ? 3 : 2;
     a.fix_p3 = (ctx->prm.fixes & SPH_FIX_ORDER3) ? 1 : 0;
-    const int threads = 256;
+    const int threads = 64;
     for (int l = (int)T.level_counts.size() - 1; l >= 0; --l) {
         a.count = T.level_counts[l];
         if (a.count == 0) continue;
