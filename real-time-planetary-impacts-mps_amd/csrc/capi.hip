@@ -449,7 +449,10 @@ int tree_reserve(sph_ctx* ctx, int64_t n_ints, const int32_t* level_counts, int 
     if (total != node_count) return ctx_fail(ctx, SPH_E_ARG, "level lists do not cover node_count nodes");
     if (level_counts[0] != 1) return ctx_fail(ctx, SPH_E_ARG, "level 0 must hold only the root");
     const double grow = 1.2; /* EXTRA_MEMORY_MULTIPLIER */
-    const int64_t list_need = (int64_t)std::max<int32_t>(max_nonlast, 1) * ctx->prm.max_unchecked_pointers;
+    /* two levels' lists in turn, or with the near-field form every level's */
+    const bool keep_lists = (ctx->prm.fixes & SPH_FIX_NEAR_FIELD) != 0;
+    const int64_t list_slots = keep_lists ? total - level_counts[n_levels - 1] : max_nonlast;
+    const int64_t list_need = std::max<int64_t>(list_slots, 1) * ctx->prm.max_unchecked_pointers;
     const bool need_realloc = n_ints > T.octree_cap || total > T.level_cap || node_count > T.node_cap ||
                               list_need > ctx->list_cap;
     if (need_realloc) {
@@ -523,7 +526,7 @@ int tree_reserve(sph_ctx* ctx, int64_t n_ints, const int32_t* level_counts, int 
             dfree(ctx->list_a);
             dfree(ctx->list_b);
             SPH_HIP_TRY(dalloc(&ctx->list_a, (size_t)cap));
-            SPH_HIP_TRY(dalloc(&ctx->list_b, (size_t)cap));
+            if (!keep_lists) SPH_HIP_TRY(dalloc(&ctx->list_b, (size_t)cap));
             ctx->list_cap = cap;
         }
     }

@@ -550,6 +550,11 @@ struct DownArgs {
      * the back, act_count[kMaxLevels] of them; null: every slot of the level */
     const int32_t* act_slots;
     const int32_t* act_count;
+    /* near-field leaves of every level in one launch: level_id and the slots
+     * count from level 1 on, and a node's parent's list is of the level
+     * before its own, from slot list_off[level - 1] on; 0: one level */
+    int all_levels;
+    int list_off[kMaxLevels];
 };
 
 struct LocalExp {
@@ -1428,7 +1433,10 @@ __device__ __forceinline__ void down_group_body(const DownArgs& a, int s, bool v
     float Lc[eNT3]; /* compensations (precision form) */
 #pragma unroll
     for (int k = 0; k < NTP; ++k) L.e[k] = Lc[k] = 0.f;
-    const int32_t* in = a.in + (live ? (int64_t)a.t.parent_slot[id] * a.maxu : 0);
+    int64_t in_slot = live ? a.t.parent_slot[id] : 0;
+    if constexpr (MODE >= 2)
+        if (live && a.all_levels) in_slot += a.list_off[inf.z - 1];
+    const int32_t* in = a.in + in_slot * a.maxu;
     /* MODE 1: branches only; MODE 2 and 3: leaves only, their M2L part and
      * then their pair sums (separate launches, so each has the registers of
      * its own path); MODE 4: leaves only, M2L and pair sums in one walk;
@@ -1525,6 +1533,19 @@ __device__ __forceinline__ void down_group_body(const DownArgs& a, int s, bool v
     }
 }
 
+/* The leaf launches: pieces of kLeafPiece consecutive workgroups go to the
+ * XCDs in turn.  The leaves come level by level, and the few of the coarse
+ * levels take hundreds of times as long as the others: an eighth of the
+ * sequence each, as the other launches', would leave them to one XCD. */
+constexpr int kLeafPiece = 16;
+__host__ __device__ __forceinline__ int leaf_grid(int blocks) {
+    return (blocks + kXcds * kLeafPiece - 1) / (kXcds * kLeafPiece) * (kXcds * kLeafPiece);
+}
+__device__ __forceinline__ int leaf_block(int b) {
+    const int x = b % kXcds, q = b / kXcds;
+    return (q / kLeafPiece * kXcds + x) * kLeafPiece + q % kLeafPiece;
+}
+
 /* One level slot per group of GS lanes.  Every slot of the level: one per
  * group, workgroups XCD-remapped.  With an active-slot list (README rule,
  * most nodes inactive): a persistent grid whose XCD x walks the x-th eighth
@@ -1537,8 +1558,15 @@ __device__ __forceinline__ void down_group_run(const DownArgs& a) {
     constexpr int GPB = 256 / GS;
     const int g = (int)threadIdx.x / GS;
     if (!a.act_slots) {
-        const int blk = xcd_block((unsigned)((a.count + GPB - 1) / GPB));
-        if (blk < 0) return;
+        const int nblk = (a.count + GPB - 1) / GPB;
+        int blk;
+        if constexpr (MODE >= 2) {
+            blk = leaf_block((int)blockIdx.x);
+            if (blk >= nblk) return;
+        } else {
+            blk = xcd_block((unsigned)nblk);
+            if (blk < 0) return;
+        }
         const int sl = blk * GPB + g;
         down_group_body<GS, NEAR, PREC, P, MODE>(a, sl, sl < a.count);
         return;
@@ -1547,11 +1575,14 @@ __device__ __forceinline__ void down_group_run(const DownArgs& a) {
     const int nl = a.act_count[0], nb = a.act_count[kMaxLevels];
     const int total = SEL == 0 ? nl + nb : (SEL == 1 ? nb : nl);
     const int nlog = (total + GPB - 1) / GPB;
-    const int per = (nlog + kXcds - 1) / kXcds;
+    const int per = MODE >= 2 ? leaf_grid(nlog) / kXcds : (nlog + kXcds - 1) / kXcds;
     const int xcd = (int)(blockIdx.x % kXcds), nper = (int)(gridDim.x / kXcds);
     for (int k = (int)(blockIdx.x / kXcds); k < per; k += nper) {
-        const int lb = xcd * per + k;
-        if (lb >= nlog) break;
+        const int lb = MODE >= 2 ? leaf_block(kXcds * k + xcd) : xcd * per + k;
+        if (lb >= nlog) {
+            if (MODE >= 2) continue; /* (a leaf's piece may end before another's) */
+            break;
+        }
         const int e = lb * GPB + g;
         const bool ok = e < total;
         const bool front = SEL == 2 || (SEL == 0 && e < nl);
@@ -1747,36 +1778,45 @@ int launch_gravity_up(sph_ctx* ctx) {
     return SPH_OK;
 }
 
-/* One level of the near-field form with GS lanes per node: branches (list
- * processing, L2L), then the leaves (balanced walk, pair sums, L2P) in one
- * or two launches; persistent over the active list, at most kDownBlocks
+/* The near-field form with GS lanes per node: one level's branches (list
+ * processing, L2L); and the leaves (balanced walk, pair sums, L2P) in one or
+ * two launches.  Persistent over the active list, at most kDownBlocks
  * workgroups, when there is one.  The near-field form runs a wave (64
  * lanes) per node: each node's walk is a chain of dependent rounds, and
  * twice the lanes halve the rounds (measured against 32 lanes: 1e6 second
  * order 107.3 -> 113.4 steps/s, third-order precision 33.9 -> 37.1, 4e6
  * learned-h + precision with individual timesteps 224.0 -> 255.0). */
 template <int GS>
-static void launch_near_level(const DownArgs& a, bool compact, bool order3, hipStream_t st) {
+static void launch_near_branches(const DownArgs& a, bool compact, bool order3, hipStream_t st) {
     const int threads = 256;
     const unsigned blocks = (unsigned)(((int64_t)a.count * GS + threads - 1) / threads);
     const dim3 g(compact ? std::min(xcd_grid(blocks), (unsigned)kDownBlocks) : xcd_grid(blocks));
     if (order3) {
+        if (a.phi) k_down_group<GS, true, true, 3, 1><<<g, threads, 0, st>>>(a);
+        else k_down_group<GS, true, false, 3, 1><<<g, threads, 0, st>>>(a);
+    } else {
+        if (a.phi) k_down_group<GS, true, true, 2, 1><<<g, threads, 0, st>>>(a);
+        else k_down_group<GS, true, false, 2, 1><<<g, threads, 0, st>>>(a);
+    }
+}
+template <int GS>
+static void launch_near_leaves(const DownArgs& a, bool compact, bool order3, hipStream_t st) {
+    const int threads = 256;
+    const unsigned blocks = (unsigned)leaf_grid((int)(((int64_t)a.count * GS + threads - 1) / threads));
+    const dim3 g(compact ? std::min(blocks, (unsigned)kDownBlocks) : blocks);
+    if (order3) {
         if (a.phi) {
-            k_down_group<GS, true, true, 3, 1><<<g, threads, 0, st>>>(a);
             k_down_leaves<GS, true, 3><<<g, threads, 0, st>>>(a);
             k_down_leaves_p2p<GS, true, 3><<<g, threads, 0, st>>>(a);
         } else {
-            k_down_group<GS, true, false, 3, 1><<<g, threads, 0, st>>>(a);
             k_down_leaves<GS, false, 3><<<g, threads, 0, st>>>(a);
             k_down_leaves_p2p<GS, false, 3><<<g, threads, 0, st>>>(a);
         }
     } else {
         if (a.phi) {
-            k_down_group<GS, true, true, 2, 1><<<g, threads, 0, st>>>(a);
             k_down_leaves<GS, true, 2><<<g, threads, 0, st>>>(a);
             k_down_leaves_p2p<GS, true, 2><<<g, threads, 0, st>>>(a);
         } else {
-            k_down_group<GS, true, false, 2, 1><<<g, threads, 0, st>>>(a);
             k_down_leaves_walk<GS, false, 2><<<g, threads, 0, st>>>(a);
         }
     }
@@ -1825,9 +1865,21 @@ int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
             SPH_HIP_TRY(hipGetLastError());
         }
     }
+    /* With the near-field form every level keeps its lists, so the leaves of
+     * all levels can wait for one launch after the last branches: a coarse
+     * level's few leaves walk for as long as a fine level's many, which then
+     * run beside them (a self-gravity step in the precision form at 2e5: 7.9 ->
+     * 4.4 ms). */
+    const bool kept = (p.fixes & SPH_FIX_NEAR_FIELD) != 0;
+    const bool together = a.near && T.level_counts.size() > 1 && T.level_counts.size() <= (size_t)kMaxLevels;
+    a.all_levels = 0;
     for (size_t l = 0; l < T.level_counts.size(); ++l) {
         int32_t* in = (l % 2 == 0) ? ctx->list_a : ctx->list_b;
         int32_t* out = (l % 2 == 0) ? ctx->list_b : ctx->list_a;
+        if (kept) {
+            in = ctx->list_a + (l > 0 ? (int64_t)T.level_offsets[l - 1] * a.maxu : 0);
+            out = ctx->list_a + (int64_t)T.level_offsets[l] * a.maxu;
+        }
         if (l == 0) {
             a.out = out;
             if (order3) k_down_root<3><<<1, 1, 0, ctx->stream>>>(a);
@@ -1847,7 +1899,8 @@ int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
                 a.act_count = T.act_count + l;
             }
             if (a.near) {
-                launch_near_level<64>(a, compact, order3, ctx->stream);
+                launch_near_branches<64>(a, compact, order3, ctx->stream);
+                if (!together) launch_near_leaves<64>(a, compact, order3, ctx->stream);
             } else {
                 /* as written: 32 lanes per node (64 measured slower at 1e6:
                  * 144.7 steps/s at every level, 151.0 at the levels of fewer
@@ -1863,6 +1916,25 @@ int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
             a.act_count = nullptr;
             k_down<<<(a.count + threads - 1) / threads, threads, 0, ctx->stream>>>(a);
         }
+        SPH_HIP_TRY(hipGetLastError());
+    }
+    if (together) {
+        const int first = T.level_offsets[1];
+        a.level_id = T.level_id + first;
+        a.count = T.level_offsets.back() + T.level_counts.back() - first;
+        a.in = ctx->list_a;
+        a.out = nullptr;
+        a.all_levels = 1;
+        for (size_t l = 0; l < T.level_counts.size(); ++l) a.list_off[l] = T.level_offsets[l];
+        if (compact) {
+            /* (level 0's counters and the levels' slots are free by now) */
+            k_level_active<<<(a.count + threads - 1) / threads, threads, 0, ctx->stream>>>(
+                a.level_id, a.count, T.mp_aux, T.node_info, T.act_slots, T.act_count);
+            SPH_HIP_TRY(hipGetLastError());
+            a.act_slots = T.act_slots;
+            a.act_count = T.act_count;
+        }
+        if (a.count > 0) launch_near_leaves<64>(a, compact, order3, ctx->stream);
         SPH_HIP_TRY(hipGetLastError());
     }
     return SPH_OK;
