@@ -1243,23 +1243,26 @@ __device__ void down_near_leaf_q(const DownArgs& a, int id, int4 inf, const Node
             int nch = 0;
             bool near_leaf = false;
             int4 near_ci = make_int4(0, 0, 0, 0);
+            int4 ch0 = make_int4(-1, -1, -1, -1), ch1 = ch0;
             if (item >= 0 && item != id) {
+                /* (all of the node's records at once: a wait per round in place of
+                 * three, 1.98 -> 1.74 ms for the leaves of 2e5 particles) */
                 const float4 b0 = a.t.far[3 * item], b1 = a.t.far[3 * item + 1], b2 = a.t.far[3 * item + 2];
+                const int4 ci = a.t.info[item];
+                ch0 = reinterpret_cast<const int4*>(a.t.child)[2 * item];
+                ch1 = reinterpret_cast<const int4*>(a.t.child)[2 * item + 1];
                 if (mac_ok(a, A, item, b0, b1, b2)) {
                     if (do_m2l) {
                         if constexpr (PREC) m2l_add_comp<P>(a, L, Lc, item, b0, b1, b2);
                         else m2l_add<P>(a, L, item, b0, b1, b2);
                     }
+                } else if (ci.x != 0) {
+                    near_leaf = true;
+                    near_ci = ci;
+                    if (PART != 1) near_p2p<PREC, NEAR_K>(a, T, nk, ci);
                 } else {
-                    const int4 ci = a.t.info[item];
-                    if (ci.x != 0) {
-                        near_leaf = true;
-                        near_ci = ci;
-                        if (PART != 1) near_p2p<PREC, NEAR_K>(a, T, nk, ci);
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 8; ++c) nch += a.t.child[8 * item + c] >= 0 ? 1 : 0;
-                    }
+                    nch = (ch0.x >= 0) + (ch0.y >= 0) + (ch0.z >= 0) + (ch0.w >= 0) + (ch1.x >= 0) + (ch1.y >= 0) +
+                          (ch1.z >= 0) + (ch1.w >= 0);
                 }
             }
             if constexpr (PART == 1) {
@@ -1292,11 +1295,10 @@ __device__ void down_near_leaf_q(const DownArgs& a, int id, int4 inf, const Node
             if (total <= QCAP - (qt - qh)) {
                 if (nch > 0) {
                     int pos = qt + before;
+                    const int ch[8] = {ch0.x, ch0.y, ch0.z, ch0.w, ch1.x, ch1.y, ch1.z, ch1.w};
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        const int ch = a.t.child[8 * item + c];
-                        if (ch >= 0) q[(pos++) % QCAP] = ch;
-                    }
+                    for (int c = 0; c < 8; ++c)
+                        if (ch[c] >= 0) q[(pos++) % QCAP] = ch[c];
                 }
                 qt += total;
             } else if (nch > 0) {
@@ -1822,6 +1824,16 @@ static void launch_near_leaves(const DownArgs& a, bool compact, bool order3, hip
     }
 }
 
+/* One level of the form as written with GS lanes per node. */
+template <int GS>
+static void launch_written_level(const DownArgs& a, bool compact, bool order3, hipStream_t st) {
+    const int threads = 256;
+    const unsigned blocks = (unsigned)(((int64_t)a.count * GS + threads - 1) / threads);
+    const dim3 g(compact ? std::min(xcd_grid(blocks), (unsigned)kDownBlocks) : xcd_grid(blocks));
+    if (order3) k_down_group<GS, false, false, 3, 0><<<g, threads, 0, st>>>(a);
+    else k_down_group<GS, false, false, 2, 0><<<g, threads, 0, st>>>(a);
+}
+
 int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
     sph_tree_dev& T = ctx->tree;
     const sph_params& p = ctx->prm;
@@ -1902,14 +1914,14 @@ int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
                 launch_near_branches<64>(a, compact, order3, ctx->stream);
                 if (!together) launch_near_leaves<64>(a, compact, order3, ctx->stream);
             } else {
-                /* as written: 32 lanes per node (64 measured slower at 1e6:
-                 * 144.7 steps/s at every level, 151.0 at the levels of fewer
-                 * than 8192 nodes, against 153.4) */
-                constexpr int GS = 32;
-                const unsigned blocks = (unsigned)(((int64_t)a.count * GS + threads - 1) / threads);
-                const dim3 g(compact ? std::min(xcd_grid(blocks), (unsigned)kDownBlocks) : xcd_grid(blocks));
-                if (order3) k_down_group<GS, false, false, 3, 0><<<g, threads, 0, ctx->stream>>>(a);
-                else k_down_group<GS, false, false, 2, 0><<<g, threads, 0, ctx->stream>>>(a);
+                /* as written: 32 lanes per node; a wave per node below 65536
+                 * particles, whose levels leave most of the GPU empty and last
+                 * as long as one node's rounds (a self-gravity step at 2e4: 429
+                 * -> 374 us; at 1e6 slower, at every level 3.20 -> 3.36 ms a
+                 * frame, at the levels of fewer than 8192 nodes 153.4 -> 151.0
+                 * steps/s) */
+                if (ctx->n < 65536) launch_written_level<64>(a, compact, order3, ctx->stream);
+                else launch_written_level<32>(a, compact, order3, ctx->stream);
             }
         } else {
             a.act_slots = nullptr;
