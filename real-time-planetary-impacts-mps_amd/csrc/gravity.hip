@@ -1824,16 +1824,6 @@ static void launch_near_leaves(const DownArgs& a, bool compact, bool order3, hip
     }
 }
 
-/* One level of the form as written with GS lanes per node. */
-template <int GS>
-static void launch_written_level(const DownArgs& a, bool compact, bool order3, hipStream_t st) {
-    const int threads = 256;
-    const unsigned blocks = (unsigned)(((int64_t)a.count * GS + threads - 1) / threads);
-    const dim3 g(compact ? std::min(xcd_grid(blocks), (unsigned)kDownBlocks) : xcd_grid(blocks));
-    if (order3) k_down_group<GS, false, false, 3, 0><<<g, threads, 0, st>>>(a);
-    else k_down_group<GS, false, false, 2, 0><<<g, threads, 0, st>>>(a);
-}
-
 int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
     sph_tree_dev& T = ctx->tree;
     const sph_params& p = ctx->prm;
@@ -1914,14 +1904,16 @@ int launch_gravity_down(sph_ctx* ctx, bool bootstrap) {
                 launch_near_branches<64>(a, compact, order3, ctx->stream);
                 if (!together) launch_near_leaves<64>(a, compact, order3, ctx->stream);
             } else {
-                /* as written: 32 lanes per node; a wave per node below 65536
-                 * particles, whose levels leave most of the GPU empty and last
-                 * as long as one node's rounds (a self-gravity step at 2e4: 429
-                 * -> 374 us; at 1e6 slower, at every level 3.20 -> 3.36 ms a
-                 * frame, at the levels of fewer than 8192 nodes 153.4 -> 151.0
-                 * steps/s) */
-                if (ctx->n < 65536) launch_written_level<64>(a, compact, order3, ctx->stream);
-                else launch_written_level<32>(a, compact, order3, ctx->stream);
+                /* as written: 32 lanes per node (64 measured slower at 1e6:
+                 * 144.7 steps/s at every level, 151.0 at the levels of fewer
+                 * than 8192 nodes, against 153.4; faster at 2e4, a
+                 * self-gravity step 429 -> 374 us, but in another order of the
+                 * sums, which later steps' smoothing lengths amplify) */
+                constexpr int GS = 32;
+                const unsigned blocks = (unsigned)(((int64_t)a.count * GS + threads - 1) / threads);
+                const dim3 g(compact ? std::min(xcd_grid(blocks), (unsigned)kDownBlocks) : xcd_grid(blocks));
+                if (order3) k_down_group<GS, false, false, 3, 0><<<g, threads, 0, ctx->stream>>>(a);
+                else k_down_group<GS, false, false, 2, 0><<<g, threads, 0, ctx->stream>>>(a);
             }
         } else {
             a.act_slots = nullptr;
