@@ -529,10 +529,14 @@ def main():
         out["pass_ms_note"] = ("gravity_down runs on its own stream, concurrently with density; its events span "
                                "that overlap, so the passes do not add up to ms_per_step")
         out["density_ms"] = round(per_pass["density"], 4)
-        # dominant kernel: the density pass is one kernel
+        # dominant kernel: the density pass is one kernel (and two small launches for what it leaves)
         dlanes = int(prm.density_lanes) if args.n >= prm.small_n_lanes else 32
         kname = (f"k_density_group<{dlanes}, {int(prm.lane_split)}, {int(prm.density_flat)}, "
                  "false, false>" if dlanes > 0 else "k_density")
+        if dlanes in (8, 32) and prm.lane_split == 0 and prm.density_flat == 0:
+            # from neighbour lists, summed in the walk's order near the fixed point only
+            gl = 16 if args.n < 65536 else 8
+            kname = f"k_density_lists<{gl}, {dlanes // gl if prm.density_stop else 0}, false, {64 // gl}>"
         # the reference algorithm's work, counted by one more sort + density
         # pass of the state after the timed steps (untimed: counting is a
         # measurement aid)
