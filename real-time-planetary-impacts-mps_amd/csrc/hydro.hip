@@ -835,8 +835,8 @@ struct FinalSums {
  * near the fixed point (29 scans) about 4k are the entries', 7k the scans'
  * roots, divisions and control, the rest the lists, deals and second pass.
  * The pass, walk -> lists, ms: with the default rule 0.72 -> 0.06 at 2e4,
- * 3.4 -> 1.36 at 1e6, 17 -> 6.1 at 4e6; near the fixed point 2.65 -> 0.41 at
- * 2e4, 3.39 -> 0.86 at 1e5, 4.94 -> 1.87 at 3e5, 11.4 -> 6.1 at 1e6.
+ * 3.4 -> 1.36 at 1e6, 17 -> 6.1 at 4e6; near the fixed point 2.65 -> 0.30 at
+ * 2e4, 3.39 -> 0.83 at 1e5, 4.94 -> 1.75 at 3e5, 11.4 -> 5.8 at 1e6.
  *
  * Particles with more entries than a list (or a bin) holds, or with a
  * position or an h that is not finite, are left to `redo`. */
@@ -2055,7 +2055,8 @@ int launch_density(sph_ctx* ctx) {
          * as fast: 1.36 against 2.2 ms at 1e6 for the same scans. */
         const int order = !p.density_stop ? 0 : (a.slots ? 16 : (ctx->n < p.small_n_lanes ? 32 : 8));
         /* 16 lanes fill the chip below 65536 particles (1 wave per SIMD at 8
-         * lanes there): 2e4 near the fixed point 0.41 ms, with 8 0.64 */
+         * lanes there): 2e4 near the fixed point 0.41 ms, with 8 0.64,
+         * before the walk queued its cells */
         const int gl = ctx->n < 65536 && (order == 0 || order == 32) ? 16 : 8;
         const unsigned waves = xcd_grid((unsigned)(((int64_t)ctx->n * gl + 63) / 64));
         const unsigned grid = a.slots ? std::min(waves, (unsigned)kListWaves) : waves;
