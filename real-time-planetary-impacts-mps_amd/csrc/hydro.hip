@@ -951,14 +951,15 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                     });
                     part = lanes_sum<64>(part);
                     const float newH = 0.5f * (hp + fminf(a.res_eta * cbrtf(lane_f(pm.w, GL * p) / part), a.max_h_len));
-                    if (g == p && fabsf(newH - hp) * hp1 > kGuessTrust) {
+                    /* (at the iteration cap no scan follows: the second pass
+                     * needs the members of this one, which no list holds) */
+                    if (g == p && count + 1 < a.max_it && fabsf(newH - hp) * hp1 > kGuessTrust) {
                         guided = redo = false;
                         h_i = h_scan = h_start;
                         h1 = 1.f / h_i;
                         reach = -1.f;
                         count++;
-                        go = count < a.max_it;
-                        density = part;
+                        go = true;
                     }
                 }
                 continue;
