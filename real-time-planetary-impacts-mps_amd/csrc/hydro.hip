@@ -971,11 +971,14 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                  * before one of its six faces enters another cell; the
                  * products are within 2^-22 of cell_box's quotients */
                 const float xyz[3] = {pm.x, pm.y, pm.z};
+                /* a particle that has stopped keeps its last scan's box,
+                 * which the second pass sums over */
+                const float hb = go ? h_i : h_scan;
                 int mn[3], mx[3];
                 float up = 3.0e38f, down = 3.0e38f, slack = 0.f;
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    const float lo = (xyz[k] - 2.f * h_i) * cells.inv, hi = (xyz[k] + 2.f * h_i) * cells.inv;
+                    const float lo = (xyz[k] - 2.f * hb) * cells.inv, hi = (xyz[k] + 2.f * hb) * cells.inv;
                     const float flo = floorf(lo), fhi = floorf(hi);
                     mn[k] = (int)flo;
                     mx[k] = (int)fhi;
@@ -985,10 +988,10 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                 }
                 up -= slack;
                 down -= slack;
-                hhi = h_i + 0.5f * cells.size * up;
-                hlo = h_i - 0.5f * cells.size * down;
+                hhi = hb + 0.5f * cells.size * up;
+                hlo = hb - 0.5f * cells.size * down;
                 if (!(fminf(up, down) > 0.f)) { /* on a cell's face: for this h alone */
-                    cell_box(make_float3(pm.x, pm.y, pm.z), cells.size, h_i, cells.mask + 1, mn, mx);
+                    cell_box(make_float3(pm.x, pm.y, pm.z), cells.size, hb, cells.mask + 1, mn, mx);
                     hhi = -1.f;
                 }
                 const int ny = mx[1] - mn[1] + 1, nz = mx[2] - mn[2] + 1;
