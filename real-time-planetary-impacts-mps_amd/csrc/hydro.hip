@@ -908,6 +908,9 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
     while (__any(go)) {
         const bool need = go && 2.f * h_i > reach;
         const bool built = __any(need);
+        /* the reference's neighbour cache: a scan over the members of the
+         * last full scan, whose box it keeps */
+        const bool cache = h_i < (float)max_h && nN < a.ne;
         if (built) {
             if (need) reach = 2.f * kReachGrow * h_i;
 #pragma unroll 1
@@ -966,14 +969,14 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
             }
         }
         if constexpr (S > 0) {
-            if (built || __any(go && !(h_i >= hlo && h_i <= hhi))) {
+            /* a particle that has stopped keeps its last scan's box too, which
+             * the second pass sums over */
+            const float hb = go && !cache ? h_i : h_scan;
+            if (built || __any(go && !(hb >= hlo && hb <= hhi))) {
                 /* the cell walk's box for this h, and how far h may move
                  * before one of its six faces enters another cell; the
                  * products are within 2^-22 of cell_box's quotients */
                 const float xyz[3] = {pm.x, pm.y, pm.z};
-                /* a particle that has stopped keeps its last scan's box,
-                 * which the second pass sums over */
-                const float hb = go ? h_i : h_scan;
                 int mn[3], mx[3];
                 float up = 3.0e38f, down = 3.0e38f, slack = 0.f;
 #pragma unroll
@@ -1024,13 +1027,12 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
         }
         const float k1 = -h1, k2 = -0.5f * h1;
         const float fac = kPi1 * h1 * h1 * h1;
-        const bool cache = h_i < (float)max_h && nN < a.ne;
         float sum;
         if (__any(go && (h_i >= 1.f || max_h > 0))) {
-            /* the reference's neighbour cache may come into play (an h of 1
-             * or more): count the members, and from the cache sum only those
-             * of the last full scan */
-            const float lim = cache ? 2.f * h_scan : 3.0e38f;
+            /* the cache may come into play (an h of 1 or more): count the
+             * members, and from the cache sum only those of the last full
+             * scan, each term with its normalisation, as the cell walk does */
+            const float h2x4 = 4.f * h_i * h_i, hb2 = cache ? 4.f * h_scan * h_scan : h2x4, hsum = h_i + h_i;
             int n = 0;
             float part[NS];
 #pragma unroll
@@ -1039,11 +1041,22 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                 for (int e = 0; e < rows[k]; ++e) {
                     const bool in = e < nb[k];
                     const float4 q = spm[in ? l.slot[g][bin_entry(k, e)] : 0];
-                    const float rr = in ? __builtin_amdgcn_sqrtf(pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z)) : 3.0e38f;
-                    n += rr <= 2.f * h_i ? 1 : 0;
-                    part[k] = add_w(part[k], rr, in && rr <= lim ? q.w : 0.f, k1, k2);
+                    const float r2 = pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z);
+                    const float rr = in ? __builtin_amdgcn_sqrtf(r2) : 3.0e38f;
+                    const bool member = in && !(r2 > hb2);
+                    n += member ? 1 : 0;
+                    if (cache) {
+                        const float w = kW_tp(rr * h1, fac);
+                        {
+#pragma clang fp contract(off)
+                            const float wm = w * q.w;
+                            part[k] += member && !(rr > hsum) ? wm : 0.f;
+                        }
+                    } else {
+                        part[k] = add_w(part[k], rr, in ? q.w : 0.f, k1, k2);
+                    }
                 }
-                part[k] *= fac;
+                part[k] *= cache ? 1.f : fac;
             }
             n = lanes_sum<GL>(n);
             if (go && !cache) nN = min(n, a.ne);
