@@ -1973,6 +1973,12 @@ int refresh_morton(sph_ctx* ctx) {
     return SPH_OK;
 }
 
+/* The particles expected within `reach` times 2 h of one, h = eta (m / rho)^(1/3). */
+static float expected_near(float eta, float reach) {
+    const float d = 2.f * reach * eta;
+    return 4.18879f * d * d * d;
+}
+
 int launch_density(sph_ctx* ctx) {
     const sph_params& p = ctx->prm;
     DensityArgs a;
@@ -2018,11 +2024,32 @@ int launch_density(sph_ctx* ctx) {
     a.slots = nullptr;
     a.nslots = nullptr;
     a.order = nullptr;
+    /* Near the fixed point (density_stop) the sums keep the order of the
+     * cell walk with this many lanes: h is iterated to 2.5e-6, its
+     * rounding noise shows in rho's and the pressure's last digits, and
+     * another order would change them (to 5e-5 of rho at 1e6).  The
+     * reference's rule stops 1e3 times earlier, and the even deal is 1.6x
+     * as fast: 1.36 against 2.2 ms at 1e6 for the same scans. */
+    const bool walk8 = !a.skip_inactive && ctx->n >= p.small_n_lanes; /* (the walk's lanes: 8, else 16 or 32) */
+    const int order = !p.density_stop ? 0 : (a.skip_inactive ? 16 : (walk8 ? 8 : 32));
     /* From lists where the particles still lie in their cells and no option
      * asks for the walk (its lane splits, its counts), for the numbers of
-     * lanes whose order the lists keep. */
+     * lanes whose order the lists keep, and where most particles' entries fit
+     * into a list: what is left is built again by a wave each, and costs more
+     * than the walk (least where a wave each still finds places).  The
+     * entries follow from resolution_eta: 84 at the default 1.2348, 136 at
+     * 1.45, 183 at 1.6, 357 at 2, 543 at 2.3.  Walk | lists, ms, on the two sides
+     * of the lines: default rule, 8 lanes, at 6e5 1.96 | 1.56 at eta 1.40 and
+     * 2.09 | 2.42 at 1.45 (at 2.0 4.46 | 6.32); 16 or 32 lanes, where every
+     * particle overflows, at 2.5e5 3.86 | 3.26 at 2.3 (within 7% of each other
+     * from 1.55 to 1.8); near the fixed point, 8 lanes, at 6e5 8.98 | 5.66 at 1.45
+     * and 9.63 | 10.0 at 1.50; 32 lanes at 1.2e5 4.81 | 3.79 at 1.55 and 5.12 |
+     * 5.44 at 1.60, at 6e4 6.95 | 6.30 at 2.0 and 10.0 | 10.1 at 2.3; a third of
+     * 6e5 active 5.64 | 3.28 at 1.50 and 6.70 | 7.49 at 1.60. */
+    const float most = order == 0 ? (walk8 ? 128.f : 600.f) : (order == 8 ? 144.f : (ctx->n < 65536 ? 600.f : 170.f));
     const bool lists = ctx->cells_fresh && p.max_nr_iterations > 0 && (p.density_stop || p.density_eta < 1.f) &&
                        !ctx->count_work && !p.lane_split && !p.density_flat &&
+                       expected_near(p.resolution_eta, kReachGrow) <= most &&
                        (a.skip_inactive ? p.list_density_lanes == 16
                                         : (ctx->n < p.small_n_lanes || p.density_lanes == 8));
     if (!lists && !a.skip_inactive && p.density_order > 0) {
@@ -2064,13 +2091,6 @@ int launch_density(sph_ctx* ctx) {
         a.redo = ctx->redo;
         a.redo_count = ctx->redo_count;
         a.clear = ctx->redo_count + 1;
-        /* Near the fixed point (density_stop) the sums keep the order of the
-         * cell walk with this many lanes: h is iterated to 2.5e-6, its
-         * rounding noise shows in rho's and the pressure's last digits, and
-         * another order would change them (to 5e-5 of rho at 1e6).  The
-         * reference's rule stops 1e3 times earlier, and the even deal is 1.6x
-         * as fast: 1.36 against 2.2 ms at 1e6 for the same scans. */
-        const int order = !p.density_stop ? 0 : (a.slots ? 16 : (ctx->n < p.small_n_lanes ? 32 : 8));
         /* 16 lanes fill the chip below 65536 particles (1 wave per SIMD at 8
          * lanes there): 2e4 near the fixed point 0.41 ms, with 8 0.64,
          * before the walk queued its cells */
@@ -2212,7 +2232,14 @@ int launch_acceleration(sph_ctx* ctx) {
     a.redo = nullptr;
     a.redo_count = nullptr;
     a.clear = nullptr;
-    if (!p.lane_split && (a.slots ? alanes == 16 : (alanes == 0 || alanes == 8 || alanes == 16))) {
+    /* Where most particles' pairs fit into a list (launch_density; 63 at the
+     * default resolution_eta, 102 at 1.45, 165 at 1.7, 268 at 2).  Walk | lists,
+     * ms: one thread at 6e5 1.37 | 0.95 at eta 1.45 and 1.44 | 1.52 at 1.50
+     * (2.65 | 10.1 at 2.0), 8 lanes at 2.5e5 2.12 | 1.21 at 1.60 and 2.11 | 4.89
+     * at 1.70, 16 lanes at 6e4 1.03 | 0.61 at 1.80 and 1.10 | 2.47 at 2.0. */
+    const float most = alanes == 0 ? 105.f : (alanes == 8 ? 144.f : 200.f);
+    if (!p.lane_split && expected_near(p.resolution_eta, 1.f) <= most &&
+        (a.slots ? alanes == 16 : (alanes == 0 || alanes == 8 || alanes == 16))) {
         /* from lists, summed in the order of the walk with that many lanes;
          * what the first launch leaves a wave each, then the walk */
         a.redo = ctx->redo;
@@ -2249,15 +2276,12 @@ int launch_acceleration(sph_ctx* ctx) {
     else                                                                                                 \
         k_acceleration_group<G, S, false>                                                                \
             <<<xcd_grid((ctx->n + (256 / (G)) - 1) / (256 / (G))), threads, 0, ctx->stream>>>(a)
-#define SPH_ACC_REST(G)                                                                                  \
-    k_acceleration_group<G, 0, true>                                                                     \
-        <<<std::min(xcd_grid((ctx->n + (256 / (G)) - 1) / (256 / (G))), (unsigned)kListBlocks), threads, 0, ctx->stream>>>(a)
     switch (asel) {
         case 4: SPH_ACC(2, 0); break;
         case 8: SPH_ACC(4, 0); break;
-        case 16: SPH_ACC_REST(8); break; /* (the lists' rest) */
+        case 16: SPH_ACC(8, 0); break;
         case 17: SPH_ACC(8, 1); break;
-        case 32: SPH_ACC_REST(16); break;
+        case 32: SPH_ACC(16, 0); break;
         case 33: SPH_ACC(16, 1); break;
         case 64: SPH_ACC(32, 0); break;
         case 65: SPH_ACC(32, 1); break;
@@ -2270,7 +2294,6 @@ int launch_acceleration(sph_ctx* ctx) {
         }
     }
 #undef SPH_ACC
-#undef SPH_ACC_REST
     SPH_HIP_TRY(hipGetLastError());
     ctx->dv_pending = true;
     return SPH_OK;
