@@ -844,6 +844,10 @@ template <int GL, int S, int P>
 __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, NearLds<GL, S, P>& l) {
     constexpr int kCap = NearLds<GL, S, P>::kCap;
     constexpr int NS = S ? S : 1, R = NearLds<GL, S, P>::kRows; /* bins per lane, and their rows in registers */
+    /* whether scans from the reference's neighbour cache are made here, or the
+     * particle left to the next launch (rare, and the code would cost the
+     * other scans of the walk's order 6%) */
+    constexpr bool kCached = S == 0 || P == 1;
     const int lane = (int)(threadIdx.x & 63), gl = lane % GL, g = P == 1 ? 0 : lane / GL;
     const bool on = index >= 0;
     if (index == 0 && gl == 0) a.time[1] = a.dt_reset;
@@ -908,9 +912,6 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
     while (__any(go)) {
         const bool need = go && 2.f * h_i > reach;
         const bool built = __any(need);
-        /* the reference's neighbour cache: a scan over the members of the
-         * last full scan, whose box it keeps */
-        const bool cache = h_i < (float)max_h && nN < a.ne;
         if (built) {
             if (need) reach = 2.f * kReachGrow * h_i;
 #pragma unroll 1
@@ -969,13 +970,13 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
             }
         }
         if constexpr (S > 0) {
-            /* a particle that has stopped keeps its last scan's box too, which
-             * the second pass sums over */
-            const float hb = go && !cache ? h_i : h_scan;
-            if (built || __any(go && !(hb >= hlo && hb <= hhi))) {
+            if (built || __any(go && !(h_i >= hlo && h_i <= hhi))) {
                 /* the cell walk's box for this h, and how far h may move
                  * before one of its six faces enters another cell; the
-                 * products are within 2^-22 of cell_box's quotients */
+                 * products are within 2^-22 of cell_box's quotients.  The last
+                 * full scan's box for a scan from the neighbour cache, and for
+                 * a particle that has stopped, whose second pass is over it */
+                const float hb = go && !(kCached && h_i < (float)max_h && nN < a.ne) ? h_i : h_scan;
                 const float xyz[3] = {pm.x, pm.y, pm.z};
                 int mn[3], mx[3];
                 float up = 3.0e38f, down = 3.0e38f, slack = 0.f;
@@ -1027,8 +1028,9 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
         }
         const float k1 = -h1, k2 = -0.5f * h1;
         const float fac = kPi1 * h1 * h1 * h1;
+        const bool cache = kCached && h_i < (float)max_h && nN < a.ne;
         float sum;
-        if (__any(go && (h_i >= 1.f || max_h > 0))) {
+        if (kCached && __any(go && (h_i >= 1.f || max_h > 0))) {
             /* the cache may come into play (an h of 1 or more): count the
              * members, and from the cache sum only those of the last full
              * scan, each term with its normalisation, as the cell walk does */
@@ -1109,6 +1111,10 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                     h_i = newH;
                     count++;
                     go = count < a.max_it;
+                    if (!kCached && go && h_i < (float)max_h) {
+                        redo = true;
+                        go = false;
+                    }
                 }
             }
             h1 = 1.f / h_i;
