@@ -1005,9 +1005,9 @@ __global__ __launch_bounds__(256) void k_down(DownArgs a) {
     if (a.t.aux[3 * id + 1].w == 0.f) return;
     const int4 inf = a.t.info[id];
     const int np = inf.x;
-    uint32_t outp = (uint32_t)s * (uint32_t)a.maxu;
-    const uint32_t maxOut = outp + (uint32_t)a.maxu;
-    if (np == 0) a.out[outp++] = id;
+    int32_t* out = a.out + (int64_t)s * a.maxu;
+    int outp = 0;
+    if (np == 0) out[outp++] = id;
     const float4 f0 = a.t.far[3 * id];
     NodeA A{f0.x, f0.y, f0.z, f0.w, a.t.aux[3 * id].w};
     LocalExp L;
@@ -1031,11 +1031,11 @@ __global__ __launch_bounds__(256) void k_down(DownArgs a) {
             for (int c = 0; c < 8; ++c) {
                 const int cid = a.t.child[8 * toScan + c];
                 if (cid == id || cid < 0) continue;
-                if (!check_add(a, A, L, cid, a.t.info[cid].x != 0 || outp == maxOut)) a.out[outp++] = cid;
+                if (!check_add(a, A, L, cid, a.t.info[cid].x != 0 || outp == a.maxu)) out[outp++] = cid;
             }
         }
     }
-    if (outp < maxOut && np == 0) a.out[outp] = -1;
+    if (outp < a.maxu && np == 0) out[outp] = -1;
     if (np == 0) {
         /* L2L (L2L.metal:90-104) to the active children */
         for (int c = 0; c < 8; ++c) l2l_child<2>(a, L, a.t.child[8 * id + c]);
@@ -1455,10 +1455,10 @@ __device__ __forceinline__ void down_group_body(const DownArgs& a, int s, bool v
                                                           near_q + (tid / GS) * QCAP);
         return;
     }
-    const uint32_t outbase = (uint32_t)s * (uint32_t)a.maxu;
+    int32_t* out = a.out + (int64_t)s * a.maxu;
     int running = 0;
     if (live && np == 0) {
-        if (lane == 0) a.out[outbase] = id;
+        if (lane == 0) out[0] = id;
         running = 1;
     }
     bool more = live;
@@ -1511,7 +1511,7 @@ __device__ __forceinline__ void down_group_body(const DownArgs& a, int s, bool v
             if (pushc) {
                 const int pos = running + __popcll(pm & ltmask);
                 if (pos >= a.maxu) take = true;
-                else a.out[outbase + (uint32_t)pos] = child;
+                else out[pos] = child;
             }
             running += __popcll(pm);
             if (take) {
@@ -1520,7 +1520,7 @@ __device__ __forceinline__ void down_group_body(const DownArgs& a, int s, bool v
             }
         }
     }
-    if (live && np == 0 && lane == 0 && running < a.maxu) a.out[outbase + (uint32_t)running] = -1;
+    if (live && np == 0 && lane == 0 && running < a.maxu) out[running] = -1;
 #pragma unroll
     for (int k = 0; k < NTP; ++k) {
         L.e[k] = group_sum<GS>(L.e[k]);
