@@ -1704,7 +1704,7 @@ struct AccelLds {
     static constexpr int kLanes = 64 / P, kTile = P == 1 ? 1 : 2;
     NearLds<GL, 1, P, !SERIAL || P == 1, false> l;
     union {
-        float term[P][kTile * kLanes * 8 + 8];
+        alignas(16) float term[P][kTile * kLanes * 8 + 8];
         WalkLds walk;
     };
 };
@@ -1729,6 +1729,8 @@ template <int GL, bool SERIAL, int P>
 __device__ __forceinline__ int accel_chunk(const AccelArgs& a, int index, AccelLds<GL, SERIAL, P>& s) {
     constexpr int kLanes = AccelLds<GL, SERIAL, P>::kLanes, kTile = AccelLds<GL, SERIAL, P>::kTile;
     constexpr int kCap = decltype(s.l)::kCap;
+    using Lds = AccelLds<GL, SERIAL, P>;
+    static_assert(offsetof(Lds, term) % 16 == 0 && sizeof(s.term[0]) % 16 == 0, "terms are float4 pairs");
     const int lane = (int)(threadIdx.x & 63), pl = lane % kLanes, g = lane / kLanes, gl = lane % GL;
     const bool on = index >= 0;
     const uint32_t ind = on ? a.sorted[index].y : 0u;
