@@ -204,6 +204,7 @@ int ctx_fail(sph_ctx* ctx, int code, const std::string& msg) {
 
 int ctx_fail_hip(sph_ctx* ctx, hipError_t e, const char* what) {
     if (ctx) ctx->err = std::string(what) + ": " + hipGetErrorString(e);
+    (void)hipGetLastError(); /* reported here, not by the next call's launches too */
     return (int)e;
 }
 
@@ -459,17 +460,23 @@ int tree_reserve(sph_ctx* ctx, int64_t n_ints, const int32_t* level_counts, int 
         /* growth: drain both streams, then reallocate (Compute.cpp:464-502) */
         SPH_HIP_TRY(hipStreamSynchronize(ctx->stream));
         SPH_HIP_TRY(hipStreamSynchronize(ctx->copy_stream));
+        /* if an allocation fails, the tree is gone with what was freed for it,
+         * and what has no capacity is allocated again by the next call */
+        bool have_tree = ctx->have_tree;
+        ctx->have_tree = false;
         if (n_ints > T.octree_cap) {
             const int64_t cap = (int64_t)(n_ints * grow) + 16;
+            T.octree_cap = 0;
             for (int k = 0; k < 2; ++k) {
                 dfree(T.octree_up[k]);
                 SPH_HIP_TRY(dalloc(&T.octree_up[k], (size_t)cap));
             }
             T.octree_cap = cap;
-            ctx->have_tree = false;
+            have_tree = false;
         }
         if (total > T.level_cap) {
             const int64_t cap = (int64_t)(total * grow) + 16;
+            T.level_cap = 0;
             for (int k = 0; k < 2; ++k) {
                 dfree(T.level_tp_up[k]);
                 SPH_HIP_TRY(dalloc(&T.level_tp_up[k], (size_t)cap));
@@ -479,10 +486,11 @@ int tree_reserve(sph_ctx* ctx, int64_t n_ints, const int32_t* level_counts, int 
             dfree(T.act_slots);
             SPH_HIP_TRY(dalloc(&T.act_slots, (size_t)cap));
             T.level_cap = cap;
-            ctx->have_tree = false;
+            have_tree = false;
         }
         if (node_count > T.node_cap) {
             const int64_t cap = (int64_t)(node_count * grow) + 16;
+            T.node_cap = 0;
             dfree(T.node_info);
             dfree(T.parent_slot);
             dfree(T.parent_level);
@@ -523,12 +531,14 @@ int tree_reserve(sph_ctx* ctx, int64_t n_ints, const int32_t* level_counts, int 
         }
         if (list_need > ctx->list_cap) {
             const int64_t cap = (int64_t)(list_need * grow) + 16;
+            ctx->list_cap = 0;
             dfree(ctx->list_a);
             dfree(ctx->list_b);
             SPH_HIP_TRY(dalloc(&ctx->list_a, (size_t)cap));
             if (!keep_lists) SPH_HIP_TRY(dalloc(&ctx->list_b, (size_t)cap));
             ctx->list_cap = cap;
         }
+        ctx->have_tree = have_tree;
     }
     /* the buffer the current tree does not use */
     *slot = ctx->have_tree ? (T.up_cur ^ 1) : T.up_cur;
