@@ -143,6 +143,12 @@ __global__ __launch_bounds__(kThreads) void k_scan_rows(uint32_t* __restrict__ t
  * ones most of the GPU, to it (alone the fill of 2^24 cells takes 21 us, at
  * the memory's rate; in the passes' shadow 8 to 10 us more than without). */
 constexpr int kFillBlocks = 512;
+/* Up to these many cells with few and with many pairs; a larger table outlasts
+ * the passes, and a launch of its own fills it faster than so few workgroups
+ * (sort_noalloc, us, alone | in the shadow: 2^27 cells 183 | 279 at 1 pair, 234 |
+ * 296 at 32768, 233 | 222 at 32769, 404 | 400 at 4e6; 2^30 cells 1368 | 2317 at
+ * 1 pair, 1431 | 1741 at 32769, 1604 | 2082 at 4e6). */
+constexpr int64_t kFillSmall = 1 << 24, kFillTiled = 1 << 27;
 struct Fill {
     uint2* se;
     int64_t count;
@@ -588,15 +594,19 @@ extern "C" int sph_sort_noalloc(const float* pos4, int32_t n, float cell_width, 
     const int cells_per_dim = 1 << cell_power;
     const int ncells = 1 << (3 * cell_power);
     uint2* se = reinterpret_cast<uint2*>(cell_se);
+    /* the cells that the sort's launches fill */
+    const bool alone = ncells > (n <= kSmallSort ? kFillSmall : kFillTiled);
+    const int64_t shared = alone ? 0 : ncells;
+    if (alone) k_fill_cells<<<(ncells + 255) / 256, 256, 0, s>>>(se, ncells);
     if (n <= kSmallSort) {
         /* the launches leave most of the GPU to the fill, a part in each */
-        const int64_t part = ncells / (passes + 1);
-        k_hash<<<(n + kThreads - 1) / kThreads + kFillBlocks, kThreads, 0, s>>>(
+        const int64_t part = shared / (passes + 1);
+        k_hash<<<(n + kThreads - 1) / kThreads + (part > 0 ? kFillBlocks : 0), kThreads, 0, s>>>(
             reinterpret_cast<const float4*>(pos4), n, cell_width, cells_per_dim, bufs[0], Fill{se, part});
-        e = small_passes(bufs, n, passes, s, se + part, ncells - part);
+        e = small_passes(bufs, n, passes, s, se + part, shared - part);
     } else {
         e = tiled_passes(bufs, n, passes, reinterpret_cast<const float4*>(pos4), cell_width, cells_per_dim, tile_hist,
-                         digit_total, s, se, ncells);
+                         digit_total, s, se, shared);
     }
     if (e != hipSuccess) return noalloc_fail((int)e, "sph_sort_noalloc: launch failed (%lld)", (long long)e);
     k_cells_bounds<<<(n + 255) / 256, 256, 0, s>>>(out, n, se);
