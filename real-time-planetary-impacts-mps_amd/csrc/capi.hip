@@ -334,8 +334,8 @@ int sph_create(const sph_params* params, const sph_ic_view* ic, const sph_eos_ta
     TRY(dalloc(&ctx->nr_iters, n));
     TRY(dalloc(&ctx->nr_order, n));
     TRY(dalloc(&ctx->redo, 2 * n));
-    TRY(dalloc(&ctx->redo_count, 2));
-    TRY(hipMemset(ctx->redo_count, 0, 8));
+    TRY(dalloc(&ctx->redo_count, 3));
+    TRY(hipMemset(ctx->redo_count, 0, 12));
     TRY(dalloc(&ctx->active, n));
     TRY(dalloc(&ctx->density_work, n));
     TRY(hipMemset(ctx->density_work, 0, 16 * n));

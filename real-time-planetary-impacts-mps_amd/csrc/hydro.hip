@@ -1271,9 +1271,11 @@ __global__ __launch_bounds__(256) void k_gather_hydro(int n, const uint2* __rest
                                                       const float* __restrict__ rho, const float* __restrict__ c,
                                                       const float* __restrict__ B, float4* __restrict__ s_posh,
                                                       float4* __restrict__ s_velb, float4* __restrict__ s_hyd,
-                                                      const uint8_t* __restrict__ mark, uint8_t epoch) {
+                                                      const uint8_t* __restrict__ mark, uint8_t epoch,
+                                                      int32_t* __restrict__ clear) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
+    if (k == 0) *clear = 0; /* (the count of slots that k_accel_lists leaves) */
     const uint2 sk = sorted[k];
     if (mark && mark[sk.x] != epoch) return;
     const uint32_t j = sk.y;
@@ -1371,11 +1373,9 @@ struct AccelArgs {
      * on the device; null: every slot */
     const int32_t* slots;
     const int32_t* nslots;
-    /* k_accel_lists: the slots it leaves to the next launch over `redo` and
-     * their count; a count that this launch clears for a later one */
+    /* k_accel_lists: the slots it leaves to k_accel_alone and their count */
     int32_t* redo;
     int32_t* redo_count;
-    int32_t* clear;
 };
 
 /* accelerations.metal:130-136: the step goal 2 CFL Gamma h / v_sig; with
@@ -1506,7 +1506,6 @@ __device__ __forceinline__ int accel_particle(const AccelArgs& a, int index) {
 /* 8 waves per SIMD (64 VGPRs, no spills) with the candidate prefetch */
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_acceleration(AccelArgs a) {
     int integerDt = 0x7FFFFFFF;
-    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if (!a.slots) {
         const int blk = xcd_block((a.n + 255) / 256);
         if (blk < 0) return;
@@ -1637,7 +1636,6 @@ __global__ __launch_bounds__(256) void k_acceleration_group(AccelArgs a) {
     constexpr int PPB = 256 / G;
     const int lane = threadIdx.x % G, g = (int)threadIdx.x / G;
     int integerDt = 0x7FFFFFFF;
-    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if constexpr (!LIST) {
         const int blk = xcd_block((a.n + PPB - 1) / PPB);
         if (blk < 0) return;
@@ -1701,13 +1699,123 @@ __device__ __forceinline__ PairTerm pair_term(const AccelArgs& a, float4 xi4, fl
  * fall on different banks. */
 template <int GL, bool SERIAL, int P>
 struct AccelLds {
-    static constexpr int kLanes = 64 / P, kTile = P == 1 ? 1 : 2;
-    NearLds<GL, 1, P, !SERIAL || P == 1, false> l;
+    static constexpr int kLanes = 64 / P, kTile = 2;
+    NearLds<GL, 1, P, !SERIAL, false> l;
     union {
         alignas(16) float term[P][kTile * kLanes * 8 + 8];
         WalkLds walk;
     };
 };
+/* The same for one particle (k_accel_alone): a part of its list at a time,
+ * which no bin overflows. */
+template <bool SERIAL>
+struct AloneBins {};
+template <>
+struct AloneBins<false> {
+    static constexpr int kBin = 224;
+    using Place = uint8_t;
+    uint16_t cell[1][kBin];
+    uint32_t bin[1][kBin / 4];
+    Place row[1][kBin][64];
+};
+template <bool SERIAL>
+struct AloneLds : AloneBins<SERIAL> {
+    static constexpr int kCap = 224;
+    int32_t slot[1][kCap];
+    alignas(16) float term[64 * 8];
+    WalkLds walk;
+};
+
+/* The terms of a particle's mycnt entries, by its LANES lanes a tile at a
+ * time into LDS, added to its sums in the order of the list: by one lane per
+ * sum (SERIAL: lane q's in sum[0], q = 0 .. 4), or by the lane of each of GL
+ * bins, the n entries of it that deal_bins gave it.  `longest`: the longest
+ * list of the wave's. */
+template <int GL, bool SERIAL, int LANES, int TILE, class Near>
+__device__ __forceinline__ void add_terms(const AccelArgs& a, Near& l, int g, float* term, int mycnt, int longest, int n,
+                                          float4 xi4, float4 vi4, float4 hyd, float hi1, float faci, float& v_sigi,
+                                          float (&sum)[5]) {
+    const int lane = (int)(threadIdx.x & 63), pl = lane % LANES;
+    int at = 0; /* bins: entries added */
+    for (int base = 0; base < longest; base += TILE * LANES) {
+        float4 xj[TILE], vj[TILE], hj[TILE];
+#pragma unroll
+        for (int e = 0; e < TILE; ++e) {
+            const int i = base + e * LANES + pl, k = i < mycnt ? l.slot[g][i] : 0;
+            xj[e] = a.s_posh[k];
+            vj[e] = a.s_velb[k];
+            hj[e] = a.s_hyd[k];
+        }
+#pragma unroll
+        for (int e = 0; e < TILE; ++e) {
+            /* past the end: terms whose products are -0, which changes no sum */
+            PairTerm t{-0.f, -0.f, -0.f, -0.f, -0.f, 0.f, 0.f};
+            if (base + e * LANES + pl < mycnt) t = pair_term(a, xi4, vi4, hyd, hi1, faci, xj[e], vj[e], hj[e], v_sigi);
+            float4* w = reinterpret_cast<float4*>(term + (e * LANES + pl) * 8);
+            w[0] = make_float4(t.x, t.y, t.z, t.u);
+            w[1] = make_float4(t.vgi, t.m, t.mr, 0.f);
+        }
+        lds_order();
+        if constexpr (SERIAL) {
+            const int q = min(pl, 4), mq = q == 4 ? 6 : 5;
+#pragma unroll 8
+            for (int e = 0; e < TILE * LANES; ++e) sum[0] = fmaf(term[e * 8 + mq], term[e * 8 + q], sum[0]);
+        } else {
+            const int end = base + TILE * LANES;
+            for (;;) {
+                int i = 0x7FFFFFFF;
+                if (at < n) i = l.row[0][at][lane];
+                const bool in = i < end;
+                if (!__any(in)) break;
+                if (in) {
+                    const float4* w = reinterpret_cast<const float4*>(term + (i - base) * 8);
+                    const float4 t = w[0], m = w[1];
+                    sum[0] = fmaf(m.y, t.x, sum[0]);
+                    sum[1] = fmaf(m.y, t.y, sum[1]);
+                    sum[2] = fmaf(m.y, t.z, sum[2]);
+                    sum[3] = fmaf(m.y, t.w, sum[3]);
+                    sum[4] = fmaf(m.z, m.x, sum[4]);
+                    ++at;
+                }
+            }
+        }
+        lds_order();
+    }
+}
+
+/* The particle's five sums and signal velocity from its lanes', in each. */
+template <int GL, bool SERIAL, int LANES>
+__device__ __forceinline__ void gather_sums(float& v_sigi, float (&sum)[5]) {
+    v_sigi = lanes_max<LANES>(v_sigi);
+    if constexpr (SERIAL) {
+        const float mine = sum[0];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) sum[q] = __shfl(mine, ((int)(threadIdx.x & 63) & ~(LANES - 1)) + q, 64);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            const float v[1] = {sum[q]};
+            sum[q] = bins_sum<GL, 1>(v);
+        }
+    }
+}
+
+/* Writes a particle's results; returns its tick step. */
+__device__ __forceinline__ int write_accel(const AccelArgs& a, uint32_t ind, float h_i, float v_sigi, const float (&sum)[5]) {
+    a.dv[ind] = make_float4(sum[0], sum[1], sum[2], 0.f);
+    a.du[ind] = sum[3];
+    a.dhdt[ind] = sum[4];
+    const float goaldt = step_goal(a, h_i, v_sigi, sum[4]);
+    int r = 0;
+    float dtCandidate = a.dt0;
+    while (dtCandidate > goaldt && r < a.r_max) {
+        dtCandidate *= 0.5f;
+        r++;
+    }
+    const int integerDt = (int)ceilf(a.dtmin * dtCandidate);
+    a.next_active[ind] = a.time[0] + integerDt;
+    return integerDt;
+}
 
 /* accelerations.metal:12-141 for the wave's P particles (64 / P lanes each),
  * from lists of their pairs: the candidates of the cell boxes that pass the
@@ -1722,7 +1830,7 @@ struct AccelLds {
  * the pass is bound by VALU issue: 4000 instructions per wave of 8 particles
  * at 1e6, half of them the test of the 13 windows of candidates.  The pass,
  * walk -> lists (with min_step's question), ms: 0.49 -> 0.19 at 2e4, 0.93 ->
- * 0.31 at 1e5, 0.77 -> 0.37 at 3e5, 1.68 -> 1.04 at 1e6, 5.4 -> 4.1 at 4e6.
+ * 0.31 at 1e5, 0.77 -> 0.37 at 3e5, 1.68 -> 1.02 at 1e6, 5.4 -> 4.1 at 4e6.
  *
  * Particles with more pairs than a list or a bin holds are left to `redo`. */
 template <int GL, bool SERIAL, int P>
@@ -1731,7 +1839,7 @@ __device__ __forceinline__ int accel_chunk(const AccelArgs& a, int index, AccelL
     constexpr int kCap = decltype(s.l)::kCap;
     using Lds = AccelLds<GL, SERIAL, P>;
     static_assert(offsetof(Lds, term) % 16 == 0 && sizeof(s.term[0]) % 16 == 0, "terms are float4 pairs");
-    const int lane = (int)(threadIdx.x & 63), pl = lane % kLanes, g = lane / kLanes, gl = lane % GL;
+    const int lane = (int)(threadIdx.x & 63), pl = lane % kLanes, g = lane / kLanes;
     const bool on = index >= 0;
     const uint32_t ind = on ? a.sorted[index].y : 0u;
     const bool act = on && a.active[ind];
@@ -1764,93 +1872,69 @@ __device__ __forceinline__ int accel_chunk(const AccelArgs& a, int index, AccelL
     const float4 hyd = act ? a.s_hyd[index] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float h_i = xi4.w, hi1 = 1.f / h_i, faci = kPi1 * hi1 * hi1 * hi1 * hi1;
     float v_sigi = 1e-12f;
-    float sum[5] = {0.f, 0.f, 0.f, 0.f, 0.f}; /* SERIAL: lane q's in sum[0], q = 0 .. 4 */
-    int at = 0;                               /* bins: entries added */
-    float* term = s.term[g];
-    for (int base = 0; base < longest; base += kTile * kLanes) {
-        float4 xj[kTile], vj[kTile], hj[kTile];
-#pragma unroll
-        for (int e = 0; e < kTile; ++e) {
-            const int i = base + e * kLanes + pl, k = i < mycnt ? s.l.slot[g][i] : 0;
-            xj[e] = a.s_posh[k];
-            vj[e] = a.s_velb[k];
-            hj[e] = a.s_hyd[k];
-        }
-#pragma unroll
-        for (int e = 0; e < kTile; ++e) {
-            /* past the end: terms whose products are -0, which changes no sum */
-            PairTerm t{-0.f, -0.f, -0.f, -0.f, -0.f, 0.f, 0.f};
-            if (base + e * kLanes + pl < mycnt) t = pair_term(a, xi4, vi4, hyd, hi1, faci, xj[e], vj[e], hj[e], v_sigi);
-            float4* w = reinterpret_cast<float4*>(term + (e * kLanes + pl) * 8);
-            w[0] = make_float4(t.x, t.y, t.z, t.u);
-            w[1] = make_float4(t.vgi, t.m, t.mr, 0.f);
-        }
-        lds_order();
-        if constexpr (SERIAL) {
-            const int q = min(pl, 4), mq = q == 4 ? 6 : 5;
-#pragma unroll 8
-            for (int e = 0; e < kTile * kLanes; ++e) sum[0] = fmaf(term[e * 8 + mq], term[e * 8 + q], sum[0]);
-        } else {
-            const int end = base + kTile * kLanes;
-            for (;;) {
-                int i = 0x7FFFFFFF;
-                if (at < nb[0]) i = s.l.row[0][at][lane];
-                const bool in = i < end;
-                if (!__any(in)) break;
-                if (in) {
-                    const float4* w = reinterpret_cast<const float4*>(term + (i - base) * 8);
-                    const float4 t = w[0], m = w[1];
-                    sum[0] = fmaf(m.y, t.x, sum[0]);
-                    sum[1] = fmaf(m.y, t.y, sum[1]);
-                    sum[2] = fmaf(m.y, t.z, sum[2]);
-                    sum[3] = fmaf(m.y, t.w, sum[3]);
-                    sum[4] = fmaf(m.z, m.x, sum[4]);
-                    ++at;
-                }
-            }
-        }
-        lds_order();
-    }
-    v_sigi = lanes_max<kLanes>(v_sigi);
-    if constexpr (SERIAL) {
-        const float mine = sum[0];
-#pragma unroll
-        for (int q = 0; q < 5; ++q) sum[q] = __shfl(mine, (lane & ~(kLanes - 1)) + q, 64);
-    } else {
-#pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            const float v[1] = {sum[q]};
-            sum[q] = bins_sum<GL, 1>(v);
-        }
-    }
+    float sum[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    add_terms<GL, SERIAL, kLanes, kTile>(a, s.l, g, s.term[g], mycnt, longest, nb[0], xi4, vi4, hyd, hi1, faci, v_sigi, sum);
+    gather_sums<GL, SERIAL, kLanes>(v_sigi, sum);
     if (pl != 0 || !act) return 0x7FFFFFFF;
     if (redo) {
         a.redo[atomicAdd(a.redo_count, 1)] = index;
         return 0x7FFFFFFF;
     }
-    a.dv[ind] = make_float4(sum[0], sum[1], sum[2], 0.f);
-    a.du[ind] = sum[3];
-    a.dhdt[ind] = sum[4];
-    const float goaldt = step_goal(a, h_i, v_sigi, sum[4]);
-    int r = 0;
-    float dtCandidate = a.dt0;
-    while (dtCandidate > goaldt && r < a.r_max) {
-        dtCandidate *= 0.5f;
-        r++;
+    return write_accel(a, ind, h_i, v_sigi, sum);
+}
+
+/* The same for one active particle by the whole wave, for any number of
+ * pairs: the list is added up whenever it is nearly full and begun anew,
+ * which leaves the order of the sums as it is. */
+template <int GL, bool SERIAL>
+__device__ __forceinline__ int accel_alone(const AccelArgs& a, int index, AloneLds<SERIAL>& s) {
+    using Lds = AloneLds<SERIAL>;
+    static_assert(offsetof(Lds, term) % 16 == 0, "terms are float4 pairs");
+    const uint32_t ind = a.sorted[index].y;
+    const float4 xi4 = a.s_posh[index], vi4 = a.s_velb[index], hyd = a.s_hyd[index];
+    const float h_i = xi4.w, hi1 = 1.f / h_i, faci = kPi1 * hi1 * hi1 * hi1 * hi1;
+    float v_sigi = 1e-12f;
+    float sum[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    int mn[3], mx[3], nc[3];
+    cell_box(make_float3(xi4.x, xi4.y, xi4.z), a.cells.cell_size, fminf(h_i, a.max_h_len), a.cells.mask + 1, mn, mx);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        mn[k] = uniform(mn[k]);
+        nc[k] = uniform(mx[k]) - mn[k] + 1;
     }
-    const int integerDt = (int)ceilf(a.dtmin * dtCandidate);
-    a.next_active[ind] = a.time[0] + integerDt;
-    return integerDt;
+    int c = 0;
+    auto add_up = [&] {
+        lds_order();
+        int nb[1] = {0};
+        if constexpr (!SERIAL) deal_bins<GL, 1, 1>(s, c, c, nc[1], nc[2], 0, nb);
+        add_terms<GL, SERIAL, 64, 1>(a, s, 0, s.term, c, c, nb[0], xi4, vi4, hyd, hi1, faci, v_sigi, sum);
+        c = 0;
+    };
+    if (nc[0] > 0 && nc[1] > 0 && nc[2] > 0)
+        wave_candidates(cell_level(a.cells, 0), a.s_posh, mn, nc[0], nc[1], nc[2], s.walk, cell_place,
+                        [&](int k, float4 q, bool valid, int tag) {
+            const bool hit = valid && !pair_skip(q, xi4.x, xi4.y, xi4.z, h_i * h_i * 4.f, q.w * q.w * 4.f);
+            const uint64_t m = __ballot(hit);
+            const int at = list_place(m, c);
+            if (hit) {
+                s.slot[0][at] = k;
+                if constexpr (!SERIAL) s.cell[0][at] = (uint16_t)tag;
+            }
+            c += (int)__popcll(m);
+            if (c > Lds::kCap - 64) add_up();
+        });
+    add_up();
+    gather_sums<GL, SERIAL, 64>(v_sigi, sum);
+    return (threadIdx.x & 63) == 0 ? write_accel(a, ind, h_i, v_sigi, sum) : 0x7FFFFFFF;
 }
 
 /* One wave per workgroup, P particles per wave, over every slot or a list as
  * k_density_lists. */
 template <int GL, bool SERIAL, bool LIST, int P = 64 / GL>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 ? 2 : 4))) void k_accel_lists(AccelArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_accel_lists(AccelArgs a) {
     __shared__ AccelLds<GL, SERIAL, P> s;
     const int g = (int)threadIdx.x / (64 / P);
     int integerDt = 0x7FFFFFFF;
-    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
     if constexpr (!LIST) {
         const int blk = xcd_block((unsigned)((a.n + P - 1) / P));
         if (blk < 0) return;
@@ -1868,6 +1952,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 ? 2 :
             integerDt = min(integerDt, accel_chunk<GL, SERIAL, P>(a, e < total ? a.slots[e] : -1, s));
         }
     }
+    min_step(a.time, integerDt);
+}
+
+/* What k_accel_lists leaves, a wave per particle. */
+template <int GL, bool SERIAL>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_accel_alone(AccelArgs a) {
+    __shared__ AloneLds<SERIAL> s;
+    const int total = *a.nslots;
+    int integerDt = 0x7FFFFFFF;
+    for (int e = (int)blockIdx.x; e < total; e += (int)gridDim.x)
+        integerDt = min(integerDt, accel_alone<GL, SERIAL>(a, uniform(a.slots[e]), s));
     min_step(a.time, integerDt);
 }
 
@@ -2229,17 +2324,16 @@ int launch_acceleration(sph_ctx* ctx) {
     if (ctx->morton_fresh)
         k_gather_hydro<true><<<(ctx->n + threads - 1) / threads, threads, 0, ctx->stream>>>(
             ctx->n, ctx->pairs_a, ctx->pos, ctx->vel, ctx->m, ctx->s_posm, ctx->s_vel, ctx->h, ctx->f, ctx->P,
-            ctx->rho, ctx->c, ctx->B, ctx->s_posh, ctx->s_velb, ctx->s_hyd, mark, epoch);
+            ctx->rho, ctx->c, ctx->B, ctx->s_posh, ctx->s_velb, ctx->s_hyd, mark, epoch, ctx->redo_count + 2);
     else
         k_gather_hydro<false><<<(ctx->n + threads - 1) / threads, threads, 0, ctx->stream>>>(
             ctx->n, ctx->pairs_a, ctx->pos, ctx->vel, ctx->m, ctx->s_posm, ctx->s_vel, ctx->h, ctx->f, ctx->P,
-            ctx->rho, ctx->c, ctx->B, ctx->s_posh, ctx->s_velb, ctx->s_hyd, mark, epoch);
+            ctx->rho, ctx->c, ctx->B, ctx->s_posh, ctx->s_velb, ctx->s_hyd, mark, epoch, ctx->redo_count + 2);
     SPH_HIP_TRY(hipGetLastError());
     const int alanes = a.slots ? p.list_accel_lanes
                                : (ctx->n < p.small_n_lanes ? (ctx->n < 65536 ? 16 : 8) : p.accel_lanes);
-    a.redo = nullptr;
-    a.redo_count = nullptr;
-    a.clear = nullptr;
+    a.redo = ctx->redo;
+    a.redo_count = ctx->redo_count + 2;
     /* Where most particles' pairs fit into a list (launch_density; 63 at the
      * default resolution_eta, 102 at 1.45, 165 at 1.7, 268 at 2).  Walk | lists,
      * ms: one thread at 6e5 1.37 | 0.95 at eta 1.45 and 1.44 | 1.52 at 1.50
@@ -2249,10 +2343,7 @@ int launch_acceleration(sph_ctx* ctx) {
     if (!p.lane_split && expected_near(p.resolution_eta, 1.f) <= most &&
         (a.slots ? alanes == 16 : (alanes == 0 || alanes == 8 || alanes == 16))) {
         /* from lists, summed in the order of the walk with that many lanes;
-         * what the first launch leaves a wave each, then the walk */
-        a.redo = ctx->redo;
-        a.redo_count = ctx->redo_count;
-        a.clear = ctx->redo_count + 1;
+         * what the first launch leaves a wave each */
         const int gl = alanes == 16 ? 16 : 8;
         const unsigned waves = xcd_grid((unsigned)(((int64_t)ctx->n * gl + 63) / 64));
         if (a.slots) k_accel_lists<16, false, true><<<std::min(waves, (unsigned)kListWaves), 64, 0, ctx->stream>>>(a);
@@ -2261,18 +2352,14 @@ int launch_acceleration(sph_ctx* ctx) {
         else k_accel_lists<8, true, false><<<waves, 64, 0, ctx->stream>>>(a);
         SPH_HIP_TRY(hipGetLastError());
         a.slots = ctx->redo;
-        a.nslots = ctx->redo_count;
-        a.redo = ctx->redo + ctx->n;
-        a.redo_count = ctx->redo_count + 1;
-        a.clear = nullptr;
-        const unsigned alone = std::min(xcd_grid(ctx->n), 2048u);
-        if (alanes == 16) k_accel_lists<16, false, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
-        else if (alanes == 8) k_accel_lists<8, false, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
-        else k_accel_lists<8, true, true, 1><<<alone, 64, 0, ctx->stream>>>(a);
-        SPH_HIP_TRY(hipGetLastError());
-        a.slots = a.redo;
         a.nslots = a.redo_count;
-        a.clear = ctx->redo_count;
+        const unsigned alone = std::min((unsigned)ctx->n, 2048u);
+        if (alanes == 16) k_accel_alone<16, false><<<alone, 64, 0, ctx->stream>>>(a);
+        else if (alanes == 8) k_accel_alone<8, false><<<alone, 64, 0, ctx->stream>>>(a);
+        else k_accel_alone<8, true><<<alone, 64, 0, ctx->stream>>>(a);
+        SPH_HIP_TRY(hipGetLastError());
+        ctx->dv_pending = true;
+        return SPH_OK;
     }
     const int asel = alanes * 2 + (p.lane_split ? 1 : 0);
     /* over a slot list the grid is persistent: at most kListBlocks workgroups */

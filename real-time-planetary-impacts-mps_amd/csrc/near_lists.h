@@ -420,6 +420,14 @@ __device__ __forceinline__ void build_near_lists(const Level& cells, const float
     lds_order();
 }
 
+/* Whether a candidate is no pair of a particle's (beyond 2 h of both, or the
+ * particle itself): the acceleration walk's own test, form for form. */
+__device__ __forceinline__ bool pair_skip(float4 q, float px, float py, float pz, float pi2x4, float qj2x4) {
+    const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    return (r2 > pi2x4 && r2 > qj2x4) || r2 < 1e-12f;
+}
+
 /* Lists of the pairs of the acceleration pass for the wave's P particles of
  * LANES lanes each: the candidates of the particle's own cell box [mn, mx]
  * (empty: none) within 2 h of either side, in the order of the cells.  The
@@ -463,13 +471,7 @@ __device__ __forceinline__ void build_pair_lists(const Level& cells, const float
         }
         c += (int)__popcll(m);
     };
-    /* the walk's own test, form for form */
-    auto skip = [](float4 q, float px, float py, float pz, float pi2x4, float qj2x4) {
-        const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
-        const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        return (r2 > pi2x4 && r2 > qj2x4) || r2 < 1e-12f;
-    };
-    if (P == 1 || (!wide && ratio <= -2.5f * groups_min(some ? -own : 0.f))) {
+    if (!wide && ratio <= -2.5f * groups_min(some ? -own : 0.f)) {
         float px[P], py[P], pz[P], ph[P];
         int pmn[P][3], pnc[P][3];
 #pragma unroll
@@ -498,7 +500,7 @@ __device__ __forceinline__ void build_pair_lists(const Level& cells, const float
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 const bool in = (tag & (1 << (15 + p))) != 0;
-                if (__any(in)) append(p, in && !skip(q, px[p], py[p], pz[p], ph[p], qj2x4), k, tag & 0x7FFF, cnt[p]);
+                if (__any(in)) append(p, in && !pair_skip(q, px[p], py[p], pz[p], ph[p], qj2x4), k, tag & 0x7FFF, cnt[p]);
             }
         });
         off = ((umn[0] - mn[0]) * ny + (umn[1] - mn[1])) * nz + (umn[2] - mn[2]);
@@ -515,7 +517,7 @@ __device__ __forceinline__ void build_pair_lists(const Level& cells, const float
             }
             wave_candidates(cells, s_posh, m, n[0], n[1], n[2], walk, cell_place,
                             [&](int k, float4 q, bool valid, int tag) {
-                append(p, valid && !skip(q, px, py, pz, ph, q.w * q.w * 4.f), k, tag, c);
+                append(p, valid && !pair_skip(q, px, py, pz, ph, q.w * q.w * 4.f), k, tag, c);
             });
 #pragma unroll
             for (int j = 0; j < P; ++j) cnt[j] = j == p ? c : cnt[j];

@@ -226,9 +226,11 @@ struct sph_ctx {
     int32_t* slot_list = nullptr;   /* sorted slots of the active particles (README rule) */
     int32_t* slot_count = nullptr;  /* their number (device) */
     bool slot_list_valid = false;   /* cleared by a sort and by a gravity pass */
-    /* slots that the first and the second launch of a list-built pass leave
-     * to the next (n each), and their counts: a pass's first launch clears the
-     * second count, its last the first one */
+    /* slots that the first and the second launch of the list-built density pass
+     * leave to the next (n each; the acceleration pass's first launch takes the
+     * first n), and their counts: the density pass's first launch clears the
+     * second count, its last the first one; the third is the acceleration
+     * pass's, cleared by its gather */
     int32_t *redo = nullptr, *redo_count = nullptr;
     sph_mlp* learned = nullptr;     /* not owned */
     sph_samples* dump = nullptr;    /* not owned */
