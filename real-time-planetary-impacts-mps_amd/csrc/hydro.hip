@@ -2226,7 +2226,8 @@ int launch_density(sph_ctx* ctx) {
         const unsigned blocks = std::min(xcd_grid((ctx->n + 7) / 8), 512u);
         if (order == 32) k_density_group<32, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
         else if (order == 16) k_density_group<16, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
-        else k_density_group<8, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
+        else if (order == 8) k_density_group<8, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
+        else k_density_group<64, 0, 0, true, false><<<std::min(xcd_grid((ctx->n + 3) / 4), 2048u), threads, 0, ctx->stream>>>(a);
         SPH_HIP_TRY(hipGetLastError());
         return SPH_OK;
     }
