@@ -842,8 +842,9 @@ struct FinalSums {
  * position or an h that is not finite, are left to `redo`. */
 template <int GL, int S, int P>
 __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, NearLds<GL, S, P>& l) {
-    constexpr int kCap = NearLds<GL, S, P>::kCap;
-    constexpr int NS = S ? S : 1, R = NearLds<GL, S, P>::kRows; /* bins per lane, and their rows in registers */
+    using Near = NearLds<GL, S, P>;
+    constexpr int kCap = Near::kCap;
+    constexpr int NS = S ? S : 1, R = Near::kRows; /* bins per lane, and their rows in registers */
     /* whether scans from the reference's neighbour cache are made here, or the
      * particle left to the next launch (rare, and the code would cost the
      * other scans of the walk's order 6%) */
@@ -889,7 +890,7 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
     float hlo = 0.f, hhi = -1.f;
     int nb[NS] = {}, rows[NS] = {};
     auto bin_entry = [&](int k, int e) -> int { /* place in the list of the k-th bin's e-th */
-        if constexpr (S > 0) return l.row[k][e][lane];
+        if constexpr (S > 0) return l.row[bin_row<S, Near>(k, e)][lane];
         return e * GL + gl;
     };
     /* entries e0 .. e0 + 3 of the k-th bin: slots, records, distances */
@@ -1005,13 +1006,9 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
                 const bool moved = go && now != shape;
                 shape = now;
                 if (built || __any(moved)) {
-                    deal_bins<GL, S, P>(l, min(mycnt, kCap), longest, ny, nz, off, nb);
-                    bool full = false;
+                    const bool full = deal_bins<GL, S, P>(l, min(mycnt, kCap), longest, ny, nz, off, nb);
 #pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        rows[k] = min(wave_max(nb[k]), NearLds<GL, S, P>::kBin);
-                        full = full || nb[k] > NearLds<GL, S, P>::kBin;
-                    }
+                    for (int k = 0; k < S; ++k) rows[k] = wave_max(nb[k]);
                     /* (any lane of the group) */
                     if (lanes_sum<GL>(full ? 1 : 0) > 0 && act) {
                         redo = true;
@@ -1712,11 +1709,11 @@ template <bool SERIAL>
 struct AloneBins {};
 template <>
 struct AloneBins<false> {
-    static constexpr int kBin = 224;
+    static constexpr int kBin = 224, kOver = 0;
     using Place = uint8_t;
     uint16_t cell[1][kBin];
     uint32_t bin[1][kBin / 4];
-    Place row[1][kBin][64];
+    Place row[kBin][64];
 };
 template <bool SERIAL>
 struct AloneLds : AloneBins<SERIAL> {
@@ -1764,7 +1761,7 @@ __device__ __forceinline__ void add_terms(const AccelArgs& a, Near& l, int g, fl
             const int end = base + TILE * LANES;
             for (;;) {
                 int i = 0x7FFFFFFF;
-                if (at < n) i = l.row[0][at][lane];
+                if (at < n) i = l.row[at][lane];
                 const bool in = i < end;
                 if (!__any(in)) break;
                 if (in) {
@@ -1861,8 +1858,8 @@ __device__ __forceinline__ int accel_chunk(const AccelArgs& a, int index, AccelL
     mycnt = redo ? 0 : mycnt;
     int nb[1] = {0};
     if constexpr (!SERIAL) {
-        deal_bins<GL, 1, P>(s.l, mycnt, longest, ny, nz, off, nb);
-        if (lanes_sum<GL>(nb[0] > decltype(s.l)::kBin ? 1 : 0) > 0 && act) {
+        const bool full = deal_bins<GL, 1, P>(s.l, mycnt, longest, ny, nz, off, nb);
+        if (lanes_sum<GL>(full ? 1 : 0) > 0 && act) {
             redo = true;
             mycnt = 0;
             nb[0] = 0;

@@ -162,7 +162,10 @@ template <int GL, int S, int P, bool WALK>
 struct NearLds<GL, S, P, true, WALK> {
     static constexpr int kCap = P == 1 ? 768 : (GL <= 8 ? 160 : 224);
     static constexpr int kRows = (P == 1 ? 64 : (S <= 1 ? 28 : 32)) / S; /* (a multiple of 4) */
-    static constexpr int kBin = P == 1 ? 192 / S : (S <= 1 ? 64 : (S == 2 ? 40 : 24));
+    static constexpr int kBin = P == 1 ? 192 / S : (S <= 1 ? 64 : (S > 2 ? 14 : (GL > 8 ? 24 : 40)));
+    /* one bin of each lane's may hold so many more: where the cells are wide
+     * (3 h or more) most of a particle's neighbours lie in a few of them */
+    static constexpr int kOver = P > 1 && (S > 2 || (S == 2 && GL > 8)) ? 40 : 0;
     using Place = typename std::conditional<(kCap > 255), uint16_t, uint8_t>::type;
     int32_t slot[P][kCap];
     /* the entries' cells, 5 bits an axis, counted from the walk's first */
@@ -173,7 +176,7 @@ struct NearLds<GL, S, P, true, WALK> {
              * compare into a mask of entries), and each bin's entries in list
              * order */
             uint32_t bin[P][kCap / 4];
-            Place row[S][kBin][64];
+            Place row[S * kBin + kOver][64];
         };
         typename std::conditional<WALK, WalkLds, NoWalk>::type walk; /* while the lists are built */
     };
@@ -526,6 +529,12 @@ __device__ __forceinline__ void build_pair_lists(const Level& cells, const float
     lds_order();
 }
 
+/* The row of the e-th entry of a lane's k-th bin. */
+template <int S, class Lds>
+__device__ __forceinline__ int bin_row(int k, int e) {
+    return Lds::kOver > 0 && e >= Lds::kBin ? (S - 1) * Lds::kBin + e : k * Lds::kBin + e;
+}
+
 /* The order of the sums of the cell walk with G = GL S lanes per particle:
  * there lane b sums the candidates of cells b, b + G, ... of the particle's
  * box in order, and the lanes' sums are added in a fixed tree.  This deals a
@@ -535,9 +544,11 @@ __device__ __forceinline__ void build_pair_lists(const Level& cells, const float
  * changes with the box: `ny`, `nz` are the box's cells in y and z and `off`
  * the position, in it, of the cell that the list's cells are counted from.
  * (An entry outside the box is beyond 2h: it adds 0 to whichever bin.)
- * n[k] = entries of the lane's k-th bin (it may exceed kBin). */
+ * n[k] = entries of the lane's k-th bin, all of them kept (bin_row); 0 for a
+ * bin with more than there is room for, of which nothing may be read, and then
+ * true. */
 template <int GL, int S, int P, class Lds>
-__device__ __forceinline__ void deal_bins(Lds& l, int have, int longest, int ny, int nz, int off, int (&n)[S]) {
+__device__ __forceinline__ bool deal_bins(Lds& l, int have, int longest, int ny, int nz, int off, int (&n)[S]) {
     constexpr uint32_t kNone = 0x40u, kMask = GL * S - 1;
     static_assert(GL * S <= 32, "cells are kept modulo 32");
     const int lane = (int)(threadIdx.x & 63), gl = lane % GL, g = P == 1 ? 0 : lane / GL;
@@ -557,6 +568,7 @@ __device__ __forceinline__ void deal_bins(Lds& l, int have, int longest, int ny,
     }
     lds_order();
     uint32_t c = 0; /* entries of the lane's bins so far, a byte each */
+    [[maybe_unused]] int over = -1; /* the bin that goes on past the others' rows */
     constexpr uint32_t kLane = (kNone | (GL - 1)) * 0x01010101u;
     const uint32_t mine = (uint32_t)gl * 0x01010101u;
     for (int w = 0; w < words; ++w) {
@@ -572,14 +584,27 @@ __device__ __forceinline__ void deal_bins(Lds& l, int have, int longest, int ny,
                 m &= m - 1u;
                 const int k = S > 1 ? (int)(bytes[byte_at(i)] / GL) : 0;
                 const int at = (int)((c >> (8 * k)) & 255u);
-                if (at < Lds::kBin) l.row[k][at][lane] = (typename Lds::Place)i;
+                if (at < Lds::kBin) l.row[k * Lds::kBin + at][lane] = (typename Lds::Place)i;
+                else if constexpr (Lds::kOver > 0) {
+                    if (over < 0) over = k;
+                    if (over == k && at < Lds::kBin + Lds::kOver)
+                        l.row[(S - 1) * Lds::kBin + at][lane] = (typename Lds::Place)i;
+                }
                 if (at < 255) c += 1u << (8 * k);
             }
         }
     }
     lds_order();
+    bool full = false;
 #pragma unroll
-    for (int k = 0; k < S; ++k) n[k] = (int)((c >> (8 * k)) & 255u);
+    for (int k = 0; k < S; ++k) {
+        n[k] = (int)((c >> (8 * k)) & 255u);
+        if (n[k] > Lds::kBin + (over == k ? Lds::kOver : 0)) {
+            n[k] = 0;
+            full = true;
+        }
+    }
+    return full;
 }
 
 /* The cell walk's tree over its G = GL S lanes (distances G/2, ..., 1); no
