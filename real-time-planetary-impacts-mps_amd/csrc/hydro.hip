@@ -817,6 +817,22 @@ struct FinalSums {
     }
 };
 
+__device__ __forceinline__ void write_density(const DensityArgs& a, uint32_t ind, const float2* table, int count, float h_i,
+                                              float density, const FinalSums& f) {
+    a.nr_iters[ind] = count;
+    const float velDiv = fabsf(f.velDiv) / density;
+    const float absCurl = sqrtf(f.cx * f.cx + f.cy * f.cy + f.cz * f.cz) / density;
+    const float fgrad = 1.f / (1.f + (h_i / (3.f * density)) * f.density_h);
+    const float2 pc = eos_sample(table, a.eos_res, a.u[ind], density, a.min_u, a.max_u, a.min_rho, a.max_rho);
+    const float bal = velDiv / (velDiv + absCurl + 1e-4f * (pc.y / h_i));
+    a.h[ind] = h_i;
+    a.rho[ind] = density;
+    a.f[ind] = fgrad;
+    a.P[ind] = pc.x;
+    a.c[ind] = pc.y;
+    a.B[ind] = bal;
+}
+
 /* density.metal:12-239 for the wave's 64 / GL particles (lane / GL), from
  * neighbour lists: the candidates within 2h (and a margin) are found once,
  * each lane keeps its share's distances and masses in registers, and every
@@ -1147,7 +1163,7 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
         t[4][k] = f.cz;
     }
     const float density_h = total(t[0]);
-    float velDiv = total(t[1]);
+    const float velDiv = total(t[1]);
     const float cx = total(t[2]), cy = total(t[3]), cz = total(t[4]);
     members = lanes_sum<GL>(members);
     const bool full = members >= a.ne;
@@ -1173,18 +1189,96 @@ __device__ __forceinline__ void density_chunk(const DensityArgs& a, int index, N
         a.redo[atomicAdd(a.redo_count, 1)] = index;
         return;
     }
-    a.nr_iters[ind] = count;
-    velDiv = fabsf(velDiv) / density;
-    const float absCurl = sqrtf(cx * cx + cy * cy + cz * cz) / density;
-    const float fgrad = 1.f / (1.f + (h_i / (3.f * density)) * density_h);
-    const float2 pc = eos_sample(table, a.eos_res, a.u[ind], density, a.min_u, a.max_u, a.min_rho, a.max_rho);
-    const float bal = velDiv / (velDiv + absCurl + 1e-4f * (pc.y / h_i));
-    a.h[ind] = h_i;
-    a.rho[ind] = density;
-    a.f[ind] = fgrad;
-    a.P[ind] = pc.x;
-    a.c[ind] = pc.y;
-    a.B[ind] = bal;
+    write_density(a, ind, table, count, h_i, density, FinalSums{density_h, velDiv, cx, cy, cz});
+}
+
+/* The same with the default rule for one active particle by the whole wave,
+ * without a list: every scan is a walk over the candidates, 64 at a time
+ * whatever cells they lie in, for particles with more neighbours than the
+ * lists of the launches before hold (the surface's, seen by an ejected
+ * particle; a core far denser than the cells).  In the cell walk the lanes
+ * take cells, and the longest lane's particles count: a twentieth of 1e6
+ * particles active, a tenth thrown out around the bodies, 8 lanes 10.6 ms, 64
+ * lanes 2.0. */
+__device__ __forceinline__ void density_alone(const DensityArgs& a, int index, WalkLds& walk) {
+    const int lane = (int)(threadIdx.x & 63);
+    const float4* __restrict__ spm = a.s_posm;
+    const float4 pm = spm[index];
+    const uint32_t ind = a.sorted[index].y;
+    const float h_start = a.h[ind];
+    float h_i = a.guess ? a.guess[index] : h_start;
+    const float far = fmaxf(fmaxf(fabsf(pm.x), fabsf(pm.y)), fabsf(pm.z)) + 4.f * (fabsf(h_i) + fabsf(h_start));
+    if (!(h_i > 0.f && h_start > 0.f && far < 1e9f * a.cells.cell_size && pm.x == pm.x && pm.y == pm.y && pm.z == pm.z)) {
+        density_group_particle<64, 0, 0, false>(a, index, lane);
+        return;
+    }
+    if (index == 0 && lane == 0) a.time[1] = a.dt_reset;
+    const float2* table = a.mat[ind] == 400 ? a.eos0 : a.eos1;
+    bool guided = a.guess != nullptr, go = true;
+    float eps_last = 3.0e38f, eps_prev = 3.0e38f, h1 = 1.f / h_i, h_scan = h_i, density = 0.f;
+    int count = 0, max_h = 0, nN = 0;
+    while (go) {
+        const bool cache = h_i < (float)max_h && nN < a.ne;
+        const float hb = cache ? h_scan : h_i, hb2 = 4.f * hb * hb, hsum = h_i + h_i, fac = kPi1 * h1 * h1 * h1;
+        const float k1 = -h1, k2 = -0.5f * h1;
+        float part = 0.f;
+        int n = 0;
+        wave_near(cell_level(a.cells, near_level(a.cells, 2.f * hb)), spm, pm.x, pm.y, pm.z, 2.f * hb, walk,
+                  [&](int, float4 q, bool valid, int) {
+            const float r2 = pair_r2(q.x - pm.x, q.y - pm.y, q.z - pm.z);
+            const bool in = valid && !(r2 > hb2);
+            const float rr = __builtin_amdgcn_sqrtf(r2);
+            n += in ? 1 : 0;
+            part = add_w(part, rr, in && (!cache || rr <= hsum) ? q.w : 0.f, k1, k2);
+        });
+        n = lanes_sum<64>(n);
+        density = lanes_sum<64>(part * fac);
+        if (!cache) {
+            nN = min(n, a.ne);
+            h_scan = h_i;
+        }
+        const float newH = 0.5f * (h_i + fminf(a.res_eta * cbrtf(pm.w / density), a.max_h_len));
+        const float eps = fabsf(newH - h_i) * h1;
+        if (guess_rejected(guided, eps, eps_last)) {
+            h_i = h_start;
+            max_h = 0;
+            eps_prev = 3.0e38f;
+            count++;
+        } else {
+            go = nr_goes_on(a.stop_rule, eps, eps_prev, a.eta);
+            eps_prev = eps;
+            if (go) {
+                max_h = (int)fmaxf((float)max_h, h_i);
+                h_i = newH;
+                count++;
+            }
+        }
+        h1 = 1.f / h_i;
+        go = go && count < a.max_it;
+    }
+    /* second pass, as density_group_particle's */
+    const float4 vi4 = a.s_vel[index];
+    const bool cached = nN < a.ne;
+    const float hb = cached ? h_scan : h_i, hb2 = 4.f * hb * hb, hsum = h_i + h_i, fac = kPi1 * h1 * h1 * h1;
+    FinalSums f;
+    float part = 0.f;
+    wave_near(cell_level(a.cells, near_level(a.cells, 2.f * hb)), spm, pm.x, pm.y, pm.z, 2.f * hb, walk,
+              [&](int k, float4 q, bool valid, int) {
+        const float dx = q.x - pm.x, dy = q.y - pm.y, dz = q.z - pm.z;
+        const float r2 = pair_r2(dx, dy, dz);
+        const float rr = __builtin_amdgcn_sqrtf(r2);
+        if (valid && !(r2 > hb2) && !(cached && rr > hsum)) {
+            f.add(rr, q.w, dx, dy, dz, a.s_vel[k], vi4, h1);
+            part += kW_tp(rr * h1, fac) * q.w;
+        }
+    });
+    if (!cached) density = (a.fix_cache ? 0.f : density) + lanes_sum<64>(part);
+    f.density_h = lanes_sum<64>(f.density_h);
+    f.velDiv = lanes_sum<64>(f.velDiv);
+    f.cx = lanes_sum<64>(f.cx);
+    f.cy = lanes_sum<64>(f.cy);
+    f.cz = lanes_sum<64>(f.cz);
+    if (lane == 0) write_density(a, ind, table, count, h_i, density, f);
 }
 
 /* One wave per workgroup, P particles per wave: consecutive sorted slots
@@ -1213,6 +1307,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P == 1 && S 
         const int e = lb * P + g;
         density_chunk<GL, S, P>(a, e < total ? a.slots[e] : -1, l);
     }
+}
+
+/* What the lists of the default rule leave, a wave per particle. */
+__global__ __launch_bounds__(64) void k_density_alone(DensityArgs a) {
+    __shared__ WalkLds walk;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0;
+    const int total = *a.nslots;
+    for (int e = (int)blockIdx.x; e < total; e += (int)gridDim.x) density_alone(a, uniform(a.slots[e]), walk);
 }
 
 /* density.metal:40-55 for the inactive particles, in original order
@@ -2224,7 +2326,7 @@ int launch_density(sph_ctx* ctx) {
         if (order == 32) k_density_group<32, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
         else if (order == 16) k_density_group<16, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
         else if (order == 8) k_density_group<8, 0, 0, true, false><<<blocks, threads, 0, ctx->stream>>>(a);
-        else k_density_group<64, 0, 0, true, false><<<std::min(xcd_grid((ctx->n + 3) / 4), 2048u), threads, 0, ctx->stream>>>(a);
+        else k_density_alone<<<std::min((unsigned)ctx->n, 2048u), 64, 0, ctx->stream>>>(a);
         SPH_HIP_TRY(hipGetLastError());
         return SPH_OK;
     }
