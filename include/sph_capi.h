@@ -114,7 +114,8 @@ typedef struct sph_params {
      * box split over that many lanes (same terms, tree-ordered sums).  At 8
      * (the default), and below small_n_lanes, the pass takes neighbour lists
      * that a wave builds in place of walking the cells scan by scan: the same
-     * terms, with density_stop 1 the same bits. */
+     * terms, with density_stop 1 the same bits (up to a resolution_eta of about
+     * 1.4, whose neighbours the lists hold; beyond it the walk). */
     int32_t density_lanes;
     /* The same for the acceleration pass (0 = one thread per particle). */
     int32_t accel_lanes;

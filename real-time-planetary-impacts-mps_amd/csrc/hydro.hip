@@ -2241,13 +2241,13 @@ int launch_density(sph_ctx* ctx) {
      * than the walk (least where a wave each still finds places).  The
      * entries follow from resolution_eta: 84 at the default 1.2348, 136 at
      * 1.45, 183 at 1.6, 357 at 2, 543 at 2.3.  Walk | lists, ms, on the two sides
-     * of the lines: default rule, 8 lanes, at 6e5 1.96 | 1.56 at eta 1.40 and
-     * 2.09 | 2.42 at 1.45 (at 2.0 4.46 | 6.32); 16 or 32 lanes, where every
-     * particle overflows, at 2.5e5 3.86 | 3.26 at 2.3 (within 7% of each other
-     * from 1.55 to 1.8); near the fixed point, 8 lanes, at 6e5 8.98 | 5.66 at 1.45
-     * and 9.63 | 10.0 at 1.50; 32 lanes at 1.2e5 4.81 | 3.79 at 1.55 and 5.12 |
-     * 5.44 at 1.60, at 6e4 6.95 | 6.30 at 2.0 and 10.0 | 10.1 at 2.3; a third of
-     * 6e5 active 5.64 | 3.28 at 1.50 and 6.70 | 7.49 at 1.60. */
+     * of the lines: default rule, 8 lanes, at 6e5 1.96 | 1.54 at eta 1.40 and
+     * 2.09 | 2.43 at 1.45 (at 2.0 4.46 | 6.32); 16 or 32 lanes, where every
+     * particle overflows, at 2.5e5 3.86 | 3.20 at 2.3 (within 5% of each other
+     * from 1.55 to 1.8); near the fixed point, 8 lanes, at 6e5 8.98 | 5.67 at 1.45
+     * and 9.63 | 10.0 at 1.50; 32 lanes at 1.2e5 4.81 | 3.85 at 1.55 and 5.12 |
+     * 5.49 at 1.60, at 6e4 6.95 | 6.34 at 2.0 and 10.0 | 10.1 at 2.3; a third of
+     * 6e5 active 5.64 | 3.27 at 1.50 and 6.70 | 7.38 at 1.60. */
     const float most = order == 0 ? (walk8 ? 128.f : 600.f) : (order == 8 ? 144.f : (ctx->n < 65536 ? 600.f : 170.f));
     const bool lists = ctx->cells_fresh && p.max_nr_iterations > 0 && (p.density_stop || p.density_eta < 1.f) &&
                        !ctx->count_work && !p.lane_split && !p.density_flat &&
@@ -2286,10 +2286,11 @@ int launch_density(sph_ctx* ctx) {
     a.redo_count = nullptr;
     a.clear = nullptr;
     if (lists) {
-        /* the particles that the first launch leaves, a wave each, then what
-         * that leaves in the cell walk: three launches, the last two small or
-         * empty (near the fixed point at 1e5 the first launch's rest took the
-         * walk 275 us, the chain of its longest; a wave each, 60 us) */
+        /* the particles that the first launch leaves, a wave each, then what no
+         * list holds, in the cell walk or (the order free) by a wave each without
+         * a list: three launches, the last two small or empty (near the fixed
+         * point at 1e5 the first launch's rest took the walk 275 us, the chain
+         * of its longest; a wave each, 60 us) */
         a.redo = ctx->redo;
         a.redo_count = ctx->redo_count;
         a.clear = ctx->redo_count + 1;
@@ -2436,9 +2437,10 @@ int launch_acceleration(sph_ctx* ctx) {
     a.redo_count = ctx->redo_count + 2;
     /* Where most particles' pairs fit into a list (launch_density; 63 at the
      * default resolution_eta, 102 at 1.45, 165 at 1.7, 268 at 2).  Walk | lists,
-     * ms: one thread at 6e5 1.37 | 0.95 at eta 1.45 and 1.44 | 1.52 at 1.50
-     * (2.65 | 10.1 at 2.0), 8 lanes at 2.5e5 2.12 | 1.21 at 1.60 and 2.11 | 4.89
-     * at 1.70, 16 lanes at 6e4 1.03 | 0.61 at 1.80 and 1.10 | 2.47 at 2.0. */
+     * ms: one thread at 6e5 1.37 | 0.83 at eta 1.45 and 1.51 | 2.26 at 1.55
+     * (2.65 | 6.08 at 2.0; at 1.5e6 2.80 | 2.21 and 3.17 | 5.73), 8 lanes at 2.5e5
+     * 2.12 | 1.02 at 1.60 and 2.11 | 2.90 at 1.70, 16 lanes at 6e4 1.03 | 0.53 at
+     * 1.80 and 1.10 | 1.46 at 2.0. */
     const float most = alanes == 0 ? 105.f : (alanes == 8 ? 144.f : 200.f);
     if (!p.lane_split && expected_near(p.resolution_eta, 1.f) <= most &&
         (a.slots ? alanes == 16 : (alanes == 0 || alanes == 8 || alanes == 16))) {

@@ -28,7 +28,8 @@
  *          node_info int4 x K (nParticles, treePointer, level, -), parent_slot int32 x K
  *          subtree_end int32 x K (first node id after the node's pre-order subtree)
  *          node_child int32 x 8K (child node ids, -1)
- *          lists a/b int32 x (max nodes of a non-last level) x max_unchecked_pointers
+ *          lists a/b int32 x (max nodes of a non-last level) x max_unchecked_pointers;
+ *                  near-field form: a alone, x (nodes of all levels but the last)
  */
 #ifndef SPH_INTERNAL_H
 #define SPH_INTERNAL_H
